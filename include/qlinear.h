@@ -247,13 +247,14 @@ int qlin_swiglu(int32_t rows, int32_t F, const void* X, int32_t x_dtype, int64_t
  * No counterpart in the reference, whose library reports its strategy through
  * rk_npu_w4a8_query / backend stats (src/npu.rs:631-661). */
 #define QLIN_PATH_GEMV_FUSED 0 /* one GEMV launch that quantizes (and normalizes) its rows itself */
-#define QLIN_PATH_GEMV 1       /* a quantize launch, then the GEMV on the quantized rows */
-#define QLIN_PATH_GEMM 2       /* a quantize launch, then the MFMA GEMM */
+#define QLIN_PATH_GEMV 1       /* a quantize launch, then the GEMV or (tile_m > 0) the wave-split-K
+                                  GEMM on the quantized rows */
+#define QLIN_PATH_GEMM 2       /* a quantize launch, then the tiled or the wave-split-K MFMA GEMM */
 typedef struct qlin_plan {
     int32_t path;       /* QLIN_PATH_* */
     int32_t launches;   /* kernel launches of the call */
     int32_t waves;      /* waves per workgroup of the GEMV / GEMM */
-    int32_t item_width; /* GEMV: output channels per item */
+    int32_t item_width; /* GEMV, wave-split-K GEMM: output channels per item / tile */
     int32_t items;      /* GEMV items, or GEMM output tiles */
     int32_t grid;       /* workgroups of the GEMV / GEMM launch */
     int32_t splits;     /* GEMM: k splits per tile */
@@ -268,16 +269,19 @@ int qlin_run_plan(const qlin_workspace* ws, const qlin_weights* weights, int32_t
  * Replaces the NPU strategy search and its on-disk cache (src/npu.rs:595-996, driven by
  * src/cli/tune.rs:10-59).  qlin_tune times, on `stream`, the variants of the path a run of
  * `rows` rows takes (decode GEMV: 4, 8 or 16 waves per channel group; GEMM: the 16x16x64
- * kernel and each tile configuration of the 32x32x32 kernel, each with 1..8 k splits),
- * checks that they all produce the same output, and records the fastest for the key (bits,
- * K, N, rows bucket, path, QLIN_SWIGLU); later runs with that key use it.  The table is
+ * kernel and each tile configuration of the 32x32x32 kernel, each with 1..8 k splits) and the
+ * planner's own wave-split-K kernel where it would run, checks that they all produce the same
+ * output, and records the fastest variant for the key (bits, K, N, rows bucket, path,
+ * QLIN_SWIGLU); later runs with that key use it, or keep the planner's kernel if that was
+ * faster still.  The table is
  * process-wide (all devices; tune on the device that runs).  QLIN_GEMV_WAVES,
  * QLIN_GEMM_SPLITS, QLIN_GEMM_KERNEL and QLIN_GEMM_CFG in the environment still take
  * precedence.  flags: 0 or QLIN_SWIGLU.  qlin_tune_load returns the number of entries read
  * (or an error code); the file is text, one entry per line: bits K N rows_bucket path swiglu
  * variant, the variant being the GEMV's waves (4, 8, 16) or, for a GEMM (path 2), splits +
  * 100 * kernel with splits 1..64 and kernel 0 (the planner's pick), 1 (16x16x64) or 2 + c
- * (32x32x32 in tile configuration c = 0..3; c = 3 for W4 only). */
+ * (32x32x32 in tile configuration c = 0..3; c = 3 for W4 only); a trailing word "planner"
+ * marks an entry slower than the planner's own kernel, which then stays in use. */
 int qlin_tune(qlin_workspace* ws, const qlin_weights* weights, int32_t rows, uint32_t flags, int32_t reps,
               void* stream);
 int qlin_tune_count(void);

@@ -41,6 +41,7 @@ struct QlinOverrides {
     int gemm_deep;        // QLIN_GEMM_DEEP, 0 / 1
     int gemm_wn;          // QLIN_GEMM_WN, 2 / 4
     int gemm_kernel;      // QLIN_GEMM_KERNEL: 16 forces the 16x16x64 kernel
+    int gemm_ks;          // QLIN_GEMM_KS: forces a wave-split-K configuration (0..19) where it fits; -2: never
     int gemm_cfg;         // QLIN_GEMM_CFG: forces the 32x32x32 kernel with tile configuration 0..3 (3: W4 only)
 };
 
@@ -85,6 +86,7 @@ QlinOverrides read_overrides() {
     o.gemm_deep = env_int("QLIN_GEMM_DEEP", -1);
     o.gemm_wn = env_int("QLIN_GEMM_WN", 4);
     o.gemm_kernel = env_int("QLIN_GEMM_KERNEL", 0);
+    o.gemm_ks = env_int("QLIN_GEMM_KS", -1);
     o.gemm_cfg = env_int("QLIN_GEMM_CFG", -1);
     return o;
 }
@@ -95,10 +97,13 @@ int current_device(int* dev) { return hipGetDevice(dev) == hipSuccess ? QLIN_OK 
 // Key: bits, K, N, rows bucket, path (0 decode GEMV with fused quantization, 1 decode GEMV
 // from quantized rows, 2 GEMM), SwiGLU.  Value: GEMV waves per group, or for a GEMM
 // k splits + kTuneKernelStep * kernel, kernel 0 the planner's own pick, 1 the 16x16x64
-// kernel, 2 + c the 32x32x32 kernel in tile configuration c (0..3; 3 for W4 only).
+// kernel, 2 + c the 32x32x32 kernel in tile configuration c (0..3; 3 for W4 only).  Plus
+// kTunePlanner where the planner's wave-split-K kernel beat every variant of the search: such
+// an entry names the best of those but leaves the choice to the planner.
 using TuneKey = std::tuple<int, int, int, int, int, int>;
 constexpr int kTuneKernelStep = 100, kTuneMaxSplits = 64;
 constexpr int kTuneKernel16 = 1, kTuneKernel32 = 2;
+constexpr int kTunePlanner = 1 << 20;
 std::map<TuneKey, int>& tune_table() {
     static std::map<TuneKey, int> t;
     return t;
@@ -107,7 +112,7 @@ std::mutex& tune_mutex() {
     static std::mutex m;
     return m;
 }
-thread_local int g_force_variant = 0;  // set by qlin_tune while it times one candidate
+thread_local int g_force_variant = 0;  // set by qlin_tune while it times one candidate (-1: the planner's own)
 std::atomic<int> g_tune_entries{0};    // entries in the table: the run path skips the lock at 0
 
 int rows_bucket(int rows) {
@@ -118,11 +123,11 @@ int rows_bucket(int rows) {
 }
 
 int tuned_variant(int bits, int K, int N, int rows, int path, bool sw) {
-    if (g_force_variant) return g_force_variant;
+    if (g_force_variant) return std::max(g_force_variant, 0);
     if (g_tune_entries.load(std::memory_order_acquire) == 0) return 0;
     std::lock_guard<std::mutex> g(tune_mutex());
     auto it = tune_table().find(TuneKey{bits, K, N, rows_bucket(rows), path, sw ? 1 : 0});
-    return it == tune_table().end() ? 0 : it->second;
+    return it == tune_table().end() || it->second >= kTunePlanner ? 0 : it->second;
 }
 
 
@@ -653,6 +658,7 @@ struct GemmPlan {
     int kernel;  // 32: the 32x32x32 kernel (tile configuration cfg), 16: the 16x16x64 kernel
     int cfg, bm, bn, threads;
     int m_tiles, n_tiles, splits, ktiles_per_split, group_m, deep, wn;
+    double est;  // estimated us of the k loop and the split exchange (0: splits forced)
 };
 
 // Kernel and tile configuration for a shape.  Measured (MI355X, four Qwen3-4B linears, M = 512
@@ -740,6 +746,7 @@ int plan_gemm(const qlin_workspace* ws, const qlin_weights* w, int rows, uint32_
                 S = t;
             }
         }
+        g.est = best;
     }
     S = std::max(1, std::min(S, ktiles));
     while (S > 1 && ((int64_t)tiles * S * slice > ws->part_ints || tiles > ws->n_counters)) --S;
@@ -794,6 +801,100 @@ int run_gemm(qlin_workspace* ws, const qlin_weights* w, int rows, const int8_t* 
     return e == hipSuccess ? QLIN_OK : QLIN_ERR_DEVICE;
 }
 
+// Wave-split-K tile configuration for quantized rows, or -1 for the GEMV / tiled GEMM.
+// A configuration is taken only where one round of workgroups covers the output (its 160 KiB
+// rings leave one workgroup per CU, and a second round costs a whole launch again: gate_up at
+// 128 rows 23.0 us in two rounds against 15.9 tiled).  Among those, the least estimated time:
+// a least-squares fit over 180 one-round measurements (five tile heights x W4 / W8 x the four
+// Qwen3-4B linears at 17..512 rows; 11% rms, and its pick within 1% of the best measured on
+// average) of a constant, the KiB a CU copies, the weight stream, the partial sums' exchange
+// and the MFMA steps.  Up to 32 rows, where the alternative is the GEMV or a one-tile-high
+// GEMM, that always won (qkv / o / gate_up / down at 16 rows 7.4 / 5.0 / 10.9 / 8.6 us ->
+// 4.2 / 4.1 / 9.3 / 7.7; at 8 rows 6.1 / 4.2 / 9.1 / 7.2 -> 4.1 / 4.0 / 9.0 / 6.5).  Above, it is
+// compared with the tiled GEMM's own estimate plus that kernel's fixed cost: qkv goes over to
+// the tiles between 256 (10.8 against 12.8 us) and 300 rows (15.1 against 13.9), down between
+// 192 (15.6 / 17.7) and 256 (17.7 / 18.0), o stays up to 512 (11.0 / 14.2).
+// Overrides of the GEMV's or the tiled GEMM's launch shape, and table entries, select those.
+constexpr double kTiledGemmFixedUs = 4.5;
+
+int pick_ks(const qlin_workspace* ws, const qlin_weights* w, int rows, int64_t ldq, uint32_t flags) {
+    const QlinOverrides& ov = ws->ov;
+    const bool sw = (flags & kFlagSwiglu) != 0;
+    if (ldq > (1 << 24)) return -1;  // row offsets of a tile are 32-bit
+    auto tile_ok = [&](int c) {
+        return gemm_ks_fits(w->bits, c) && !(sw && gemm_ks_tile(c).nb % 2);
+    };
+    if (ov.gemm_ks >= 0 && ov.gemm_ks < kKsConfigs) return tile_ok(ov.gemm_ks) ? ov.gemm_ks : -1;
+    if (ov.gemm_ks == -2 || ov.gemm_kernel || ov.gemm_cfg >= 0 || ov.gemm_splits > 0 || ov.gemv_waves > 0 ||
+        ov.gemv_grid >= 0 || ov.gemv_item_width > 0)
+        return -1;
+    const bool gemv = gemv_ok(ws, w, rows);
+    if (tuned_variant(w->bits, w->K, w->N, rows, gemv ? 1 : 2, sw)) return -1;
+    const int cols = sw ? w->N / 2 : w->N, steps = w->Kp / 128;
+    int best = -1;
+    double best_us = 1e30;
+    for (int c = 0; c < kKsConfigs; ++c) {
+        if (!tile_ok(c)) continue;
+        const KsTile t = gemm_ks_tile(c);
+        const int tm = 16 * t.mf, tc = sw ? 8 * t.nb : 16 * t.nb;
+        if ((int64_t)((rows + tm - 1) / tm) * ((cols + tc - 1) / tc) > ws->cu_count) continue;
+        const double own = (steps + t.wk - 1) / t.wk;  // k steps of the busiest wave
+        const double us = 1.7 + 0.0059 * t.wk * own * (2 * t.mf + t.nb * (w->bits == 4 ? 1 : 2)) +
+                          0.25e-6 * ((double)w->N * w->wrow) + 0.0087 * t.wk * t.mf * t.nb +
+                          0.0066 * own * t.wk * t.mf * t.nb;
+        if (us < best_us) {
+            best_us = us;
+            best = c;
+        }
+    }
+    if (best < 0 || rows <= kGemvMaxRowsWide) return best;
+    GemmPlan g;
+    if (plan_gemm(ws, w, rows, flags, &g)) return -1;
+    return best_us < g.est + kTiledGemmFixedUs ? best : -1;
+}
+
+int run_ks(qlin_workspace* ws, const qlin_weights* w, int cfg, int rows, const int8_t* q, int64_t ldq, const float* s,
+           void* C, int c_kind, int64_t ldc, uint32_t flags, hipStream_t st, const ResidualArgs* res) {
+    const KsTile t = gemm_ks_tile(cfg);
+    const bool sw = (flags & kFlagSwiglu) != 0;
+    const int tc = sw ? 8 * t.nb : 16 * t.nb;
+    GemmParams p{};
+    if (res) {
+        p.R = res->R;
+        p.ldr = res->ldr;
+        p.r_f16 = res->r_f16;
+        p.rmult = res->mult;
+    }
+    p.W = w->W;
+    p.wscale = w->scales;
+    p.wrow = w->wrow;
+    p.K = w->K;
+    p.Kp = w->Kp;
+    p.N = w->N;
+    p.Np = w->Np;
+    p.M = rows;
+    p.q = q;
+    p.ldq = ldq;
+    p.s = s;
+    p.C = C;
+    p.ldc = ldc;
+    p.c_kind = c_kind;
+    p.flags = flags;
+    p.m_tiles = (rows + 16 * t.mf - 1) / (16 * t.mf);
+    p.n_tiles = ((sw ? w->N / 2 : w->N) + tc - 1) / tc;
+    return launch_gemm_ks(p, w->bits, cfg, st) == hipSuccess ? QLIN_OK : QLIN_ERR_DEVICE;
+}
+
+// The linear on rows already quantized: wave-split-K GEMM, GEMV or tiled GEMM.
+int run_rows(qlin_workspace* ws, const qlin_weights* w, int rows, const int8_t* q, int64_t ldq, const float* s, void* C,
+             int c_kind, int64_t ldc, uint32_t flags, hipStream_t st, const ResidualArgs* res = nullptr) {
+    const int ks = pick_ks(ws, w, rows, ldq, flags);
+    if (ks >= 0) return run_ks(ws, w, ks, rows, q, ldq, s, C, c_kind, ldc, flags, st, res);
+    if (gemv_ok(ws, w, rows))
+        return run_gemv(ws, w, rows, nullptr, 0, 0, nullptr, 0.0f, q, ldq, s, C, c_kind, ldc, flags, st, res);
+    return run_gemm(ws, w, rows, q, ldq, s, C, c_kind, ldc, flags, st, res);
+}
+
 int check_run(const qlin_workspace* ws, const qlin_weights* w, int rows, uint32_t flags) {
     if (!ws || !w || rows <= 0 || rows > ws->max_rows) return QLIN_ERR_PARAM;
     if (w->Kp > ws->max_kp || w->Np > ws->max_np) return QLIN_ERR_PARAM;
@@ -831,10 +932,7 @@ int run_impl(qlin_workspace* ws, const qlin_weights* w, int rows, const void* A,
     qp.eps = eps;
     qp.flags = flags;
     if (launch_quant(qp, rows, st) != hipSuccess) return QLIN_ERR_DEVICE;
-    if (gemv_ok(ws, w, rows))
-        return run_gemv(ws, w, rows, nullptr, 0, 0, nullptr, 0.0f, ws->q, w->Kp, ws->s, C, c_dtype == QLIN_F16,
-                        ldc, flags, st, res);
-    return run_gemm(ws, w, rows, ws->q, w->Kp, ws->s, C, c_dtype == QLIN_F16 ? 1 : 0, ldc, flags, st, res);
+    return run_rows(ws, w, rows, ws->q, w->Kp, ws->s, C, c_dtype == QLIN_F16, ldc, flags, st, res);
 }
 
 int run_host(qlin_workspace* ws, const qlin_weights* w, int rows, const float* A, float* C, uint32_t flags) {
@@ -899,10 +997,7 @@ int qlin_gemm_i32(qlin_workspace* ws, const qlin_weights* w, int32_t rows, const
     if (!q || !acc || ldq < w->Kp || ldq % 16 || (reinterpret_cast<uintptr_t>(q) & 15) || ldacc < w->N)
         return QLIN_ERR_PARAM;
     ws->last = (hipStream_t)stream;
-    if (gemv_ok(ws, w, rows))
-        return run_gemv(ws, w, rows, nullptr, 0, 0, nullptr, 0.0f, q, ldq, nullptr, acc, 2, ldacc, 0,
-                        (hipStream_t)stream);
-    return run_gemm(ws, w, rows, q, ldq, nullptr, acc, 2, ldacc, 0, (hipStream_t)stream);
+    return run_rows(ws, w, rows, q, ldq, nullptr, acc, 2, ldacc, 0, (hipStream_t)stream);
 }
 
 int qlin_run_quantized(qlin_workspace* ws, const qlin_weights* w, int32_t rows, const int8_t* q, int64_t ldq,
@@ -914,10 +1009,7 @@ int qlin_run_quantized(qlin_workspace* ws, const qlin_weights* w, int32_t rows, 
         return QLIN_ERR_PARAM;
     hipStream_t st = (hipStream_t)stream;
     ws->last = st;
-    if (gemv_ok(ws, w, rows))
-        return run_gemv(ws, w, rows, nullptr, 0, 0, nullptr, 0.0f, q, ldq, s, C, c_dtype == QLIN_F16, ldc,
-                        flags, st);
-    return run_gemm(ws, w, rows, q, ldq, s, C, c_dtype == QLIN_F16 ? 1 : 0, ldc, flags, st);
+    return run_rows(ws, w, rows, q, ldq, s, C, c_dtype == QLIN_F16, ldc, flags, st);
 }
 
 int qlin_run_plan(const qlin_workspace* ws, const qlin_weights* w, int32_t rows, const void* A, int64_t lda,
@@ -936,6 +1028,18 @@ int qlin_run_plan(const qlin_workspace* ws, const qlin_weights* w, int32_t rows,
         return QLIN_OK;
     }
     out->launches = 2;
+    const int ks = pick_ks(ws, w, rows, w->Kp, flags);
+    if (ks >= 0) {
+        const KsTile t = gemm_ks_tile(ks);
+        const int tc = (flags & kFlagSwiglu) ? 8 * t.nb : 16 * t.nb, cols = (flags & kFlagSwiglu) ? w->N / 2 : w->N;
+        out->path = gemv_ok(ws, w, rows) ? QLIN_PATH_GEMV : QLIN_PATH_GEMM;
+        out->waves = t.wk;
+        out->tile_m = 16 * t.mf;
+        out->tile_n = out->item_width = tc;
+        out->items = out->grid = ((rows + 16 * t.mf - 1) / (16 * t.mf)) * ((cols + tc - 1) / tc);
+        out->splits = 1;
+        return QLIN_OK;
+    }
     if (gemv_ok(ws, w, rows)) {
         const GemvPlan g = plan_gemv(ws, w, rows, false, false, flags);
         out->path = QLIN_PATH_GEMV;
@@ -1322,6 +1426,10 @@ int qlin_tune(qlin_workspace* ws, const qlin_weights* w, int32_t rows, uint32_t 
     const bool fused = gemv_fusable(ws, w, rows, A, w->K, nullptr, flags);
     const int path = fused ? 0 : (gemv_ok(ws, w, rows) ? 1 : 2);
     std::vector<int> cand;
+    g_force_variant = -1;
+    if (!fused && pick_ks(ws, w, rows, w->Kp, flags) >= 0) cand.push_back(-1);
+    g_force_variant = 0;
+    const size_t own = cand.size();  // the planner's own choice comes first where it is not one of the variants
     if (path < 2) {
         for (int v : {4, 8, 16})
             if (!fused || gemv_can_fuse(rows, w->K, v, false)) cand.push_back(v);
@@ -1362,10 +1470,10 @@ int qlin_tune(qlin_workspace* ws, const qlin_weights* w, int32_t rows, uint32_t 
             if (!rc && (pass == 0 || ms < ms_min[i])) ms_min[i] = ms;
         }
     }
-    size_t bi = 0;
-    for (size_t i = 1; i < cand.size(); ++i)
+    size_t bi = own;
+    for (size_t i = own + 1; i < cand.size(); ++i)
         if (ms_min[i] < ms_min[bi]) bi = i;
-    const int best = rc || cand.empty() ? 0 : cand[bi];
+    const int best = rc || cand.size() <= own ? 0 : cand[bi] + (own && ms_min[0] <= ms_min[bi] ? kTunePlanner : 0);
     g_force_variant = 0;
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
@@ -1395,10 +1503,11 @@ int qlin_tune_save(const char* path) {
     std::FILE* f = std::fopen(path, "w");
     if (!f) return QLIN_ERR_PARAM;
     std::lock_guard<std::mutex> g(tune_mutex());
-    std::fprintf(f, "# qlinear variant table: bits K N rows_bucket path swiglu variant\n");
+    std::fprintf(f, "# qlinear variant table: bits K N rows_bucket path swiglu variant [planner]\n");
     for (auto& kv : tune_table())
-        std::fprintf(f, "%d %d %d %d %d %d %d\n", std::get<0>(kv.first), std::get<1>(kv.first), std::get<2>(kv.first),
-                     std::get<3>(kv.first), std::get<4>(kv.first), std::get<5>(kv.first), kv.second);
+        std::fprintf(f, "%d %d %d %d %d %d %d%s\n", std::get<0>(kv.first), std::get<1>(kv.first), std::get<2>(kv.first),
+                     std::get<3>(kv.first), std::get<4>(kv.first), std::get<5>(kv.first), kv.second % kTunePlanner,
+                     kv.second >= kTunePlanner ? " planner" : "");
     return std::fclose(f) == 0 ? QLIN_OK : QLIN_ERR_PARAM;
 }
 
@@ -1412,7 +1521,8 @@ int qlin_tune_load(const char* path) {
     while (std::fgets(line, sizeof line, f)) {
         if (line[0] == '#' || line[0] == '\n') continue;
         int b = 0, K = 0, N = 0, r = 0, path_ = -1, swg = -1, v = 0;
-        const bool parsed = std::sscanf(line, "%d %d %d %d %d %d %d", &b, &K, &N, &r, &path_, &swg, &v) == 7;
+        char word[9] = "";
+        const bool parsed = std::sscanf(line, "%d %d %d %d %d %d %d %8s", &b, &K, &N, &r, &path_, &swg, &v, word) >= 7;
         // a GEMM entry: 1..64 splits and a kernel field of 0..5 (5, the 256 x 192 tiles, W4 only)
         const bool ok_gemm = v % kTuneKernelStep >= 1 && v % kTuneKernelStep <= kTuneMaxSplits &&
                              v / kTuneKernelStep <= kTuneKernel32 + (b == 4 ? 3 : 2);
@@ -1422,7 +1532,8 @@ int qlin_tune_load(const char* path) {
             rc = QLIN_ERR_PARAM;
             break;
         }
-        tune_table()[TuneKey{b, K, N, r, path_, swg}] = v;
+        // a trailing "planner": the planner's own kernel was faster than this variant
+        tune_table()[TuneKey{b, K, N, r, path_, swg}] = v + (std::strcmp(word, "planner") == 0 ? kTunePlanner : 0);
         ++n;
     }
     g_tune_entries.store((int)tune_table().size(), std::memory_order_release);

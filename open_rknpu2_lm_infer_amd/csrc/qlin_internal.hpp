@@ -139,6 +139,14 @@ struct GemmTileCfg {
 };
 GemmTileCfg gemm32_tile(int bits, int cfg);
 hipError_t launch_gemm32(const GemmParams& p, int bits, int cfg, hipStream_t stream);
+// Tile configuration of the wave-split-K GEMM: row fragments and channel blocks of 16, waves along k.
+struct KsTile {
+    int mf, nb, wk;
+};
+constexpr int kKsConfigs = 20;
+KsTile gemm_ks_tile(int cfg);
+bool gemm_ks_fits(int bits, int cfg);  // two stages of every wave's ring fit the LDS
+hipError_t launch_gemm_ks(const GemmParams& p, int bits, int cfg, hipStream_t stream);
 hipError_t launch_swiglu(int rows, int F, const void* X, int x_f16, int64_t ldx, void* Y, int y_f16, int64_t ldy,
                          hipStream_t stream);
 hipError_t launch_pack_w4(const int8_t* codes_nk, int N, int K, int Np, int Kp, uint8_t* out,
