@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "qlin_gemv_parts.hpp"
 #include "qlin_rows.hpp"
 
 namespace qlin {
@@ -85,8 +86,8 @@ __global__ __launch_bounds__(kRowThreads) void quant_rows_kernel(QuantParams p) 
 // waves (the least latency per row); with many rows, 64 (one wave per row, many rows
 // resident per CU) keeps more rows' sequential norm chains in flight at once, where
 // 256-thread rows left three of four waves idle during the sum (M = 4096, K = 2560 with
-// RMSNorm: 19.6 -> 14.6 us).  Many RMSNorm rows of up to 8 chunks per lane with 16-byte
-// aligned weights take quant_norm_wave_kernel instead.  Rows of up to kStageBytes take this path (the
+// RMSNorm: 19.6 -> 14.6 us).  RMSNorm rows in the reference's chain order with 16-byte
+// aligned weights take quant_norm_block_kernel or quant_norm_wave_kernel instead.  Rows of up to kStageBytes take this path (the
 // default 64 KiB workgroup LDS limit, less the static reduction words).  Needs
 // K % 8 == 0 and a 16-byte aligned row (16-byte copies).
 constexpr int kStageBytes = 60 * 1024;
@@ -217,22 +218,25 @@ __global__ __launch_bounds__(NT) void quant_rows_staged_kernel(QuantParams p) {
 // two-byte reads; with 16 rows per CU the two-byte reads held the sum at ~3.6 us per row
 // against ~1.1 us alone).  The 8-element pad puts the 16 chains' reads, and the two
 // chains written by one store instruction, in different banks.  Needs K % 512 == 0
-// (trips of four reads).  Called by all 64 lanes; the result is valid in lane 0.
-__device__ __forceinline__ float cm_sumsq_neon16(const _Float16* cm, int K) {
+// (trips of four reads; f32 rows the same with 4 elements per read and K % 256 == 0).
+// Called by all 64 lanes; the result is valid in lane 0.
+template <typename T>
+__device__ __forceinline__ float cm_sumsq_neon16(const T* cm, int K) {
+    constexpr int E = 16 / sizeof(T);  // values per 16-byte read
     const int lane = threadIdx.x & 63, j = lane & 15;
-    const int ls = K / 16 + 8;
+    const int ls = K / 16 + E;
     float acc = 0.0f;
     if (lane < 16) {
         const uint4* c = reinterpret_cast<const uint4*>(cm + j * ls);
-        for (int r = 0; r < K / 128; r += 4) {
+        for (int r = 0; r < K / (16 * E); r += 4) {
             uint4 v[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) v[u] = c[r + u];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const _Float16* h = reinterpret_cast<const _Float16*>(&v[u]);
+                const T* h = reinterpret_cast<const T*>(&v[u]);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
+                for (int e = 0; e < E; ++e) {
                     const float f = (float)h[e];
                     acc = __builtin_fmaf(f, f, acc);
                 }
@@ -243,6 +247,124 @@ __device__ __forceinline__ float cm_sumsq_neon16(const _Float16* cm, int K) {
     const float tj = (acc + b) + (c + d);
     const float t1 = __shfl(tj, 1, 64), t2 = __shfl(tj, 2, 64), t3 = __shfl(tj, 3, 64);
     return (tj + t1) + (t2 + t3);
+}
+
+// RMSNorm rows up to about a thousand, one workgroup per row with one or two 16-byte chunks
+// per thread: latency is all there is (one row per CU or a few), so every load, the row's and
+// its RMSNorm weights', is issued at once and held in registers, and the row goes to LDS
+// chain-major, in the layout of cm_sumsq_neon16, for the serial norm sum.  The staged kernel
+// loads the weights again in both passes, a dependent round trip each, and its sum reads two
+// bytes at a time.  Same arithmetic, value for value.  Per launch in a graph (us, staged ->
+// this): K = 2560 fp16 at 24 / 128 / 512 rows 5.4 / 5.5 / 6.1 -> 3.7 / 3.8 / 4.3, f32 at 300
+// rows 5.8 -> 4.5; K = 9728 fp16 at 128 rows 10.5 -> 7.1.  Rows without RMSNorm gained
+// nothing from it (2.8 -> 2.6 us at 128 rows, 4.0 -> 4.4 at 1024) and keep their kernel.
+// Needs K % (64 E) == 0 (whole trips of the sum), a 16-byte aligned row and weights, an
+// 8-byte aligned q with ldq % 8 == 0.
+template <typename T, int NC>
+__global__ __launch_bounds__(1024) void quant_norm_block_kernel(QuantParams p) {
+    extern __shared__ __align__(16) uint8_t stage[];
+    __shared__ float red[17];
+    __shared__ int bad;
+    constexpr int E = 16 / sizeof(T);
+    const int row = blockIdx.x, t = threadIdx.x, nt = blockDim.x;
+    const T* x = reinterpret_cast<const T*>(p.A) + (int64_t)row * p.lda;
+    const int nchunks = p.K / E;
+    // (a clamped chunk repeats the last one: harmless for the max and the finiteness test,
+    // and its LDS copy writes the same values to the same place)
+    uint4 raw[NC];
+    float v[NC][E];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) raw[i] = reinterpret_cast<const uint4*>(x)[min(t + nt * i, nchunks - 1)];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const float4* g = reinterpret_cast<const float4*>(p.gamma + (int64_t)min(t + nt * i, nchunks - 1) * E);
+#pragma unroll
+        for (int h = 0; h < E / 4; ++h) {
+            const float4 a = g[h];
+            v[i][4 * h] = a.x;
+            v[i][4 * h + 1] = a.y;
+            v[i][4 * h + 2] = a.z;
+            v[i][4 * h + 3] = a.w;
+        }
+    }
+    if (t < 16) red[t] = 0.0f;
+    if (t == 0) bad = 0;
+    constexpr int CPP = 16 / E;  // chunks per position of the 16 chains
+    const int ls = p.K / 16 + E;
+    T* cm = reinterpret_cast<T*>(stage);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int c = min(t + nt * i, nchunks - 1);
+        const T* h = reinterpret_cast<const T*>(&raw[i]);
+#pragma unroll
+        for (int e = 0; e < E; ++e) cm[(E * (c % CPP) + e) * ls + c / CPP] = h[e];
+    }
+    lds_barrier();
+    if (t < 64) {
+        const float sum = cm_sumsq_neon16(cm, p.K);
+        if (t == 0) red[16] = 1.0f / __builtin_sqrtf(sum / (float)p.K + p.eps);
+    }
+    lds_barrier();
+    const float nscale = red[16];
+    // absmax (after the norm) and finiteness (of the input, from its bit patterns)
+    float m = 0.0f;
+    uint32_t top = 0;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const T* e = reinterpret_cast<const T*>(&raw[i]);
+        constexpr uint32_t kAbs = sizeof(T) == 2 ? 0x7FFF7FFFu : 0x7FFFFFFFu;
+        const uint32_t w[4] = {raw[i].x & kAbs, raw[i].y & kAbs, raw[i].z & kAbs, raw[i].w & kAbs};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) top = max(top, sizeof(T) == 2 ? max(w[j] & 0xFFFFu, w[j] >> 16) : w[j]);
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            const float xv = lds_ld(e, j);
+            v[i][j] = (xv * nscale) * v[i][j];
+            m = fmaxf(m, fabsf(v[i][j]));
+        }
+    }
+    m = wave_max_nonneg(m);
+    if ((t & 63) == 0) red[t >> 6] = m;
+    if (top >= (sizeof(T) == 2 ? 0x7C00u : 0x7F800000u)) bad = 1;
+    lds_barrier();
+    m = lane_value(rows_max_lanes<16, 1>(red), 0);
+    const int f = bad;
+    const float s = qscale_from_absmax(m);
+    const float inv = 1.0f / s;
+    const bool rne = (p.flags & kFlagRne) != 0;
+    const bool fast = !f && __builtin_isfinite(s);  // finite row: the short rounding sequence
+    int8_t* qrow = p.q + (int64_t)row * p.ldq;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int c = t + nt * i;
+        if (c < nchunks) {
+            if constexpr (E == 8) {
+                uint32_t w0, w1;
+                quant8(v[i], inv, rne, fast, w0, w1);
+                *reinterpret_cast<uint2*>(qrow + c * E) = make_uint2(w0, w1);
+            } else {
+                *reinterpret_cast<uint32_t*>(qrow + c * E) = quant4(v[i], inv, rne, fast);
+            }
+        }
+    }
+    for (int k0 = p.K + 8 * t; k0 < p.ldq; k0 += 8 * nt) *reinterpret_cast<uint2*>(qrow + k0) = make_uint2(0, 0);
+    if (t == 0) {
+        p.s[row] = s;
+        if (f && p.err) atomicOr(p.err, 1u);
+    }
+}
+
+template <typename T>
+static bool launch_quant_block(const QuantParams& p, int rows, hipStream_t stream) {
+    constexpr int E = 16 / sizeof(T);
+    const int chunks = p.K / E;
+    const size_t lds = (size_t)(p.K + 16 * E) * sizeof(T);
+    if (chunks > 2048 || lds > (size_t)kStageBytes || (p.flags & kFlagNormSeq) || p.K % (64 * E))
+        return false;
+    const int nc = chunks > 1024 ? 2 : 1, threads = ((chunks + nc - 1) / nc + 63) / 64 * 64;
+    if (nc == 1) quant_norm_block_kernel<T, 1><<<dim3(rows), dim3(threads), lds, stream>>>(p);
+    else quant_norm_block_kernel<T, 2><<<dim3(rows), dim3(threads), lds, stream>>>(p);
+    return true;
 }
 
 template <typename T, int NC, bool CM>
@@ -487,6 +609,12 @@ hipError_t launch_quant(const QuantParams& p, int rows, hipStream_t stream) {
     const bool qvec = ((reinterpret_cast<uintptr_t>(p.q) & 7) == 0) && (p.ldq % 8 == 0);
     if (vec && qvec && !p.gamma) {
         const bool ok = p.a_f16 ? launch_quant_reg<__half>(p, rows, stream) : launch_quant_reg<float>(p, rows, stream);
+        if (ok) return hipGetLastError();
+    }
+    // RMSNorm rows below 1024: a workgroup per row (K = 2560 fp16 at 512 rows 6.1 -> 4.3 us; at
+    // 2048 rows it takes 9.3 against the one-wave-per-row kernel's 8.0)
+    if (vec && qvec && rows < 1024 && p.gamma && (reinterpret_cast<uintptr_t>(p.gamma) & 15) == 0) {
+        const bool ok = p.a_f16 ? launch_quant_block<__half>(p, rows, stream) : launch_quant_block<float>(p, rows, stream);
         if (ok) return hipGetLastError();
     }
     if (vec && qvec && row_bytes <= (size_t)kStageBytes) {

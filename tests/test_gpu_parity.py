@@ -186,6 +186,30 @@ def test_rmsnorm_quantize_many_rows_nonfinite(oracle, dtype, K):
     assert np.array_equal(s.cpu().numpy().view(np.uint32)[finite], so.view(np.uint32)[finite])
 
 
+# RMSNorm rows below 1024, a workgroup per row: one and two 16-byte chunks per thread (K up to
+# 8192 fp16 / 4096 f32, then twice that), the smallest K of each type, a K whose chunks do not
+# fill the last wave, the longest rows, one row and the most rows of its range
+@pytest.mark.parametrize("dtype,K,M", [
+    (torch.float16, 512, 3), (torch.float16, 2560, 1023), (torch.float16, 8192, 2), (torch.float16, 8704, 5),
+    (torch.float16, 16384, 1), (torch.float32, 256, 3), (torch.float32, 2560, 300), (torch.float32, 4096, 1),
+    (torch.float32, 4352, 5), (torch.float32, 8192, 2)])
+def test_rmsnorm_quantize_row_per_workgroup(oracle, dtype, K, M):
+    x = synth.activations(M + 3, K, seed=K + 5, device="cpu", dist="student_t3").to(dtype)
+    x[M, 7], x[M + 1, K - 1], x[M + 2] = float("nan"), float("-inf"), 0.0
+    gam = synth.gamma(K, seed=K + 2, device="cpu")
+    ldq = roundup(K, 256) + 256
+    for rows in (M, M + 3):
+        for flags, mode in ((0, oracle.ROUND_AWAY), (ql.QLIN_ROUND_HALF_EVEN, oracle.ROUND_EVEN)):
+            err = torch.zeros(1, dtype=torch.int32, device=DEV)
+            q, s = ql.quantize(x[:rows].to(DEV), ldq=ldq, gamma=gam.to(DEV), eps=1e-6, flags=flags, err=err)
+            torch.cuda.synchronize()
+            qo, so, bad = oracle.quantize(oracle.rmsnorm(x[:rows].float().numpy(), gam.numpy(), 1e-6, "neon16"), mode)
+            assert int(err.item()) == (1 if rows > M else 0) and bad == (2 if rows > M else 0)
+            fine = np.isfinite(x[:rows].float().numpy()).all(1)
+            assert np.array_equal(s.cpu().numpy().view(np.uint32)[fine], so.view(np.uint32)[fine])
+            assert np.array_equal(q.cpu().numpy()[:, :K], qo) and not q.cpu().numpy()[:, K:].any()
+
+
 # ------------------------------------------------------------------ integer accumulators
 
 
