@@ -45,7 +45,8 @@ COMMON = [
 # compiler's AGPR heuristics the two-tile unrolled k loop re-shuffled the accumulator
 # registers on every iteration.
 FILE_FLAGS = {"qlin_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-              "qlin_gemm_ks.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+              "qlin_gemm_ks.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+              "qlin_gemm_pp.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 ROOT = os.path.dirname(HERE)
 TEST_SRC = os.path.join(ROOT, "tests", "cpp", "npu_backend_test.cpp")

@@ -41,7 +41,8 @@ struct QlinOverrides {
     int gemm_deep;        // QLIN_GEMM_DEEP, 0 / 1
     int gemm_wn;          // QLIN_GEMM_WN, 2 / 4
     int gemm_kernel;      // QLIN_GEMM_KERNEL: 16 forces the 16x16x64 kernel
-    int gemm_ks;          // QLIN_GEMM_KS: forces a wave-split-K configuration (0..19) where it fits; -2: never
+    int gemm_ks;          // QLIN_GEMM_KS: forces a wave-split-K configuration (0..19); -2: never that kernel
+    int gemm_pp;          // QLIN_GEMM_PP: forces an alternating-waves configuration (0..7); -2: never
     int gemm_cfg;         // QLIN_GEMM_CFG: forces the 32x32x32 kernel with tile configuration 0..3 (3: W4 only)
 };
 
@@ -87,6 +88,7 @@ QlinOverrides read_overrides() {
     o.gemm_wn = env_int("QLIN_GEMM_WN", 4);
     o.gemm_kernel = env_int("QLIN_GEMM_KERNEL", 0);
     o.gemm_ks = env_int("QLIN_GEMM_KS", -1);
+    o.gemm_pp = env_int("QLIN_GEMM_PP", -1);
     o.gemm_cfg = env_int("QLIN_GEMM_CFG", -1);
     return o;
 }
@@ -98,7 +100,7 @@ int current_device(int* dev) { return hipGetDevice(dev) == hipSuccess ? QLIN_OK 
 // from quantized rows, 2 GEMM), SwiGLU.  Value: GEMV waves per group, or for a GEMM
 // k splits + kTuneKernelStep * kernel, kernel 0 the planner's own pick, 1 the 16x16x64
 // kernel, 2 + c the 32x32x32 kernel in tile configuration c (0..3; 3 for W4 only).  Plus
-// kTunePlanner where the planner's wave-split-K kernel beat every variant of the search: such
+// kTunePlanner where the planner's own kernel beat every variant of the search: such
 // an entry names the best of those but leaves the choice to the planner.
 using TuneKey = std::tuple<int, int, int, int, int, int>;
 constexpr int kTuneKernelStep = 100, kTuneMaxSplits = 64;
@@ -801,63 +803,122 @@ int run_gemm(qlin_workspace* ws, const qlin_weights* w, int rows, const int8_t* 
     return e == hipSuccess ? QLIN_OK : QLIN_ERR_DEVICE;
 }
 
-// Wave-split-K tile configuration for quantized rows, or -1 for the GEMV / tiled GEMM.
-// A configuration is taken only where one round of workgroups covers the output (its 160 KiB
-// rings leave one workgroup per CU, and a second round costs a whole launch again: gate_up at
-// 128 rows 23.0 us in two rounds against 15.9 tiled).  Among those, the least estimated time:
-// a least-squares fit over 180 one-round measurements (five tile heights x W4 / W8 x the four
-// Qwen3-4B linears at 17..512 rows; 11% rms, and its pick within 1% of the best measured on
-// average) of a constant, the KiB a CU copies, the weight stream, the partial sums' exchange
-// and the MFMA steps.  Up to 32 rows, where the alternative is the GEMV or a one-tile-high
-// GEMM, that always won (qkv / o / gate_up / down at 16 rows 7.4 / 5.0 / 10.9 / 8.6 us ->
-// 4.2 / 4.1 / 9.3 / 7.7; at 8 rows 6.1 / 4.2 / 9.1 / 7.2 -> 4.1 / 4.0 / 9.0 / 6.5).  Above, it is
-// compared with the tiled GEMM's own estimate plus that kernel's fixed cost: qkv goes over to
-// the tiles between 256 (10.8 against 12.8 us) and 300 rows (15.1 against 13.9), down between
-// 192 (15.6 / 17.7) and 256 (17.7 / 18.0), o stays up to 512 (11.0 / 14.2).
-// Overrides of the GEMV's or the tiled GEMM's launch shape, and table entries, select those.
-constexpr double kTiledGemmFixedUs = 4.5;
+// Launch of a linear on quantized rows by the wave-split-K or the alternating-waves GEMM.
+struct RowsPlan {
+    enum Kind { kOther, kWaveSplitK, kAlternating } kind;  // kOther: the GEMV or the tiled GEMM
+    int cfg, bm, tc, waves;  // tile rows, output channels
+    int m_tiles, n_tiles;
+};
 
-int pick_ks(const qlin_workspace* ws, const qlin_weights* w, int rows, int64_t ldq, uint32_t flags) {
+RowsPlan rows_tiles(RowsPlan::Kind kind, int cfg, int bm, int bn, int waves, const qlin_weights* w, int rows, bool sw) {
+    RowsPlan r{kind, cfg, bm, sw ? bn / 2 : bn, waves, 0, 0};
+    r.m_tiles = (rows + r.bm - 1) / r.bm;
+    r.n_tiles = ((sw ? w->N / 2 : w->N) + r.tc - 1) / r.tc;
+    return r;
+}
+
+// Which kernel takes quantized rows.
+//
+// Wave-split-K: a configuration is taken only where one round of workgroups covers the output
+// (its 160 KiB rings leave one workgroup per CU, and a second round costs a whole launch
+// again: gate_up at 128 rows 23.0 us in two rounds against 15.9 tiled).  Among those, the
+// least estimated time: a least-squares fit over 180 one-round measurements (five tile heights
+// x W4 / W8 x the four Qwen3-4B linears at 17..512 rows; 11% rms, and its pick within 1% of
+// the best measured on average) of a constant, the KiB a CU copies, the weight stream, the
+// partial sums' exchange and the MFMA steps.  Up to 32 rows, where the alternative is the GEMV
+// or a one-tile-high GEMM, that always won (qkv / o / gate_up / down at 16 rows 7.4 / 5.0 /
+// 10.9 / 8.6 us -> 4.2 / 4.1 / 9.3 / 7.7; at 8 rows 6.1 / 4.2 / 9.1 / 7.2 -> 4.1 / 4.0 / 9.0 /
+// 6.5).
+//
+// Above 32 rows it is compared with the alternating-waves GEMM (rounds of tiles at the
+// measured us per k step and per tile of each configuration) and with the tiled GEMM's own
+// estimate plus that kernel's fixed cost, whose split K keeps few tiles of a long K ahead:
+// down at 300 / 512 rows 19.8 / 21.7 us, unsplit 31.7 / 33.1.  o keeps the wave-split-K kernel
+// up to 512 rows (11.0 us; 16.0 alternating), qkv up to 256 (10.8; 12.1); qkv at 300 / 512 /
+// 1024 / 4096 rows tiled -> alternating 14.2 / 14.8 / 23.2 / 72.5 -> 12.0 / 12.6 / 19.6 / 58.1.
+// The 0.9 leaves split cases within the estimates' error (o at 640 rows: 15.8 tiled, 16.2
+// alternating) where they were.  W4 gate_up at 300 / 512 / 1024 / 4096 rows: 29.3 / 33.0 / 58.0 /
+// 195 -> 23.4 / 29.0 / 54.0 / 164; W8 qkv at 4096 112.7 -> 72.0, gate_up 300 -> 218.
+//
+// Overrides of the GEMV's or the tiled GEMM's launch shape, and table entries, select those.
+RowsPlan plan_rows(const qlin_workspace* ws, const qlin_weights* w, int rows, int64_t ldq, uint32_t flags) {
+    const RowsPlan other{RowsPlan::kOther, 0, 0, 0, 0, 0, 0};
     const QlinOverrides& ov = ws->ov;
-    const bool sw = (flags & kFlagSwiglu) != 0;
-    if (ldq > (1 << 24)) return -1;  // row offsets of a tile are 32-bit
-    auto tile_ok = [&](int c) {
-        return gemm_ks_fits(w->bits, c) && !(sw && gemm_ks_tile(c).nb % 2);
+    const bool sw = (flags & kFlagSwiglu) != 0, w4 = w->bits == 4;
+    if (ldq > (1 << 22)) return other;  // row offsets of a tile are 32-bit
+    auto ks_ok = [&](int c) { return gemm_ks_fits(w->bits, c) && !(sw && gemm_ks_tile(c).nb % 2); };
+    auto pp_ok = [&](int c) {
+        const PpTile t = gemm_pp_tile(c);
+        return (w4 ? t.w4 : t.w8) && (sw ? t.swiglu : t.plain);
     };
-    if (ov.gemm_ks >= 0 && ov.gemm_ks < kKsConfigs) return tile_ok(ov.gemm_ks) ? ov.gemm_ks : -1;
-    if (ov.gemm_ks == -2 || ov.gemm_kernel || ov.gemm_cfg >= 0 || ov.gemm_splits > 0 || ov.gemv_waves > 0 ||
-        ov.gemv_grid >= 0 || ov.gemv_item_width > 0)
-        return -1;
-    const bool gemv = gemv_ok(ws, w, rows);
-    if (tuned_variant(w->bits, w->K, w->N, rows, gemv ? 1 : 2, sw)) return -1;
-    const int cols = sw ? w->N / 2 : w->N, steps = w->Kp / 128;
-    int best = -1;
-    double best_us = 1e30;
-    for (int c = 0; c < kKsConfigs; ++c) {
-        if (!tile_ok(c)) continue;
+    auto ks_plan = [&](int c) {
         const KsTile t = gemm_ks_tile(c);
-        const int tm = 16 * t.mf, tc = sw ? 8 * t.nb : 16 * t.nb;
-        if ((int64_t)((rows + tm - 1) / tm) * ((cols + tc - 1) / tc) > ws->cu_count) continue;
+        return rows_tiles(RowsPlan::kWaveSplitK, c, 16 * t.mf, 16 * t.nb, t.wk, w, rows, sw);
+    };
+    auto pp_plan = [&](int c) {
+        const PpTile t = gemm_pp_tile(c);
+        return rows_tiles(RowsPlan::kAlternating, c, t.bm, t.bn, 8, w, rows, sw);
+    };
+    if (ov.gemm_ks >= 0 && ov.gemm_ks < kKsConfigs) return ks_ok(ov.gemm_ks) ? ks_plan(ov.gemm_ks) : other;
+    if (ov.gemm_pp >= 0 && ov.gemm_pp < kPpConfigs) return pp_ok(ov.gemm_pp) ? pp_plan(ov.gemm_pp) : other;
+    if (ov.gemm_kernel || ov.gemm_cfg >= 0 || ov.gemm_splits > 0 || ov.gemv_waves > 0 || ov.gemv_grid >= 0 ||
+        ov.gemv_item_width > 0)
+        return other;
+    if (tuned_variant(w->bits, w->K, w->N, rows, gemv_ok(ws, w, rows) ? 1 : 2, sw)) return other;
+    const int steps = w->Kp / 128;
+    RowsPlan best = other;
+    double best_us = 1e30;
+    for (int c = 0; c < kKsConfigs && ov.gemm_ks != -2; ++c) {
+        if (!ks_ok(c)) continue;
+        const RowsPlan r = ks_plan(c);
+        if ((int64_t)r.m_tiles * r.n_tiles > ws->cu_count) continue;
+        const KsTile t = gemm_ks_tile(c);
         const double own = (steps + t.wk - 1) / t.wk;  // k steps of the busiest wave
-        const double us = 1.7 + 0.0059 * t.wk * own * (2 * t.mf + t.nb * (w->bits == 4 ? 1 : 2)) +
+        const double us = 1.7 + 0.0059 * t.wk * own * (2 * t.mf + t.nb * (w4 ? 1 : 2)) +
                           0.25e-6 * ((double)w->N * w->wrow) + 0.0087 * t.wk * t.mf * t.nb +
                           0.0066 * own * t.wk * t.mf * t.nb;
         if (us < best_us) {
             best_us = us;
-            best = c;
+            best = r;
         }
     }
-    if (best < 0 || rows <= kGemvMaxRowsWide) return best;
+    if (rows <= kGemvMaxRowsWide) return best;
     GemmPlan g;
-    if (plan_gemm(ws, w, rows, flags, &g)) return -1;
-    return best_us < g.est + kTiledGemmFixedUs ? best : -1;
+    if (plan_gemm(ws, w, rows, flags, &g)) return other;
+    const int cus = ws->cu_count, rounds = (g.m_tiles * g.n_tiles + cus - 1) / cus;
+    // W4: two workgroups of the tiled GEMM share a CU, W8: one; the estimate's k step is W4's.
+    // Splitting more tiles than half the CUs gained nothing (o at 1024 rows, 160 tiles: 23.3 us
+    // with 1 or 2 splits).
+    const bool split = g.splits > 1 && 2 * g.m_tiles * g.n_tiles <= cus;
+    double tiled_us = split ? (w4 ? 1.0 : 1.15) * g.est + 4.5
+                            : (w4 ? 0.45 : 0.60) * steps + 6.0;
+    if (rounds > 1) tiled_us *= w4 ? 0.8 * rounds : rounds;
+    if (g.kernel == 32) tiled_us = 1e30;  // its tiles are the alternating kernel's, slower on every grid
+    if (best_us >= tiled_us) {
+        best = other;
+        best_us = (split ? 0.9 : 1.0) * tiled_us;
+    }
+    for (int c = 0; c < kPpConfigs && ov.gemm_pp != -2; ++c) {
+        if (!pp_ok(c)) continue;
+        const RowsPlan r = pp_plan(c);
+        const PpTile t = gemm_pp_tile(c);
+        const int n = (int)std::min<int64_t>(((int64_t)r.m_tiles * r.n_tiles + cus - 1) / cus, 1 << 20);
+        // a tile's fixed part grows with the share of CUs that store at once, and shrinks for
+        // the later rounds, whose first copies run under the previous tile's epilogue
+        const double load = 1.0 + 0.4 * r.m_tiles * r.n_tiles / ((double)n * cus);
+        const double us = n * steps * (w4 ? t.step_us : t.step8_us) + (0.25 + 0.75 * n) * t.tile_us * load +
+                          0.12e-6 * ((double)w->N * w->wrow);
+        if (us < best_us) {
+            best_us = us;
+            best = r;
+        }
+    }
+    return best;
 }
 
-int run_ks(qlin_workspace* ws, const qlin_weights* w, int cfg, int rows, const int8_t* q, int64_t ldq, const float* s,
-           void* C, int c_kind, int64_t ldc, uint32_t flags, hipStream_t st, const ResidualArgs* res) {
-    const KsTile t = gemm_ks_tile(cfg);
-    const bool sw = (flags & kFlagSwiglu) != 0;
-    const int tc = sw ? 8 * t.nb : 16 * t.nb;
+int run_planned(qlin_workspace* ws, const qlin_weights* w, const RowsPlan& r, int rows, const int8_t* q, int64_t ldq,
+                const float* s, void* C, int c_kind, int64_t ldc, uint32_t flags, hipStream_t st,
+                const ResidualArgs* res) {
     GemmParams p{};
     if (res) {
         p.R = res->R;
@@ -880,16 +941,19 @@ int run_ks(qlin_workspace* ws, const qlin_weights* w, int cfg, int rows, const i
     p.ldc = ldc;
     p.c_kind = c_kind;
     p.flags = flags;
-    p.m_tiles = (rows + 16 * t.mf - 1) / (16 * t.mf);
-    p.n_tiles = ((sw ? w->N / 2 : w->N) + tc - 1) / tc;
-    return launch_gemm_ks(p, w->bits, cfg, st) == hipSuccess ? QLIN_OK : QLIN_ERR_DEVICE;
+    p.m_tiles = r.m_tiles;
+    p.n_tiles = r.n_tiles;
+    p.group_m = std::max(1, std::min(r.m_tiles, ws->ov.gemm_group_m));
+    const hipError_t e = r.kind == RowsPlan::kWaveSplitK ? launch_gemm_ks(p, w->bits, r.cfg, st)
+                                                         : launch_gemm_pp(p, w->bits, r.cfg, ws->cu_count, st);
+    return e == hipSuccess ? QLIN_OK : QLIN_ERR_DEVICE;
 }
 
-// The linear on rows already quantized: wave-split-K GEMM, GEMV or tiled GEMM.
+// The linear on rows already quantized.
 int run_rows(qlin_workspace* ws, const qlin_weights* w, int rows, const int8_t* q, int64_t ldq, const float* s, void* C,
              int c_kind, int64_t ldc, uint32_t flags, hipStream_t st, const ResidualArgs* res = nullptr) {
-    const int ks = pick_ks(ws, w, rows, ldq, flags);
-    if (ks >= 0) return run_ks(ws, w, ks, rows, q, ldq, s, C, c_kind, ldc, flags, st, res);
+    const RowsPlan r = plan_rows(ws, w, rows, ldq, flags);
+    if (r.kind != RowsPlan::kOther) return run_planned(ws, w, r, rows, q, ldq, s, C, c_kind, ldc, flags, st, res);
     if (gemv_ok(ws, w, rows))
         return run_gemv(ws, w, rows, nullptr, 0, 0, nullptr, 0.0f, q, ldq, s, C, c_kind, ldc, flags, st, res);
     return run_gemm(ws, w, rows, q, ldq, s, C, c_kind, ldc, flags, st, res);
@@ -1028,15 +1092,14 @@ int qlin_run_plan(const qlin_workspace* ws, const qlin_weights* w, int32_t rows,
         return QLIN_OK;
     }
     out->launches = 2;
-    const int ks = pick_ks(ws, w, rows, w->Kp, flags);
-    if (ks >= 0) {
-        const KsTile t = gemm_ks_tile(ks);
-        const int tc = (flags & kFlagSwiglu) ? 8 * t.nb : 16 * t.nb, cols = (flags & kFlagSwiglu) ? w->N / 2 : w->N;
+    const RowsPlan r = plan_rows(ws, w, rows, w->Kp, flags);
+    if (r.kind != RowsPlan::kOther) {
         out->path = gemv_ok(ws, w, rows) ? QLIN_PATH_GEMV : QLIN_PATH_GEMM;
-        out->waves = t.wk;
-        out->tile_m = 16 * t.mf;
-        out->tile_n = out->item_width = tc;
-        out->items = out->grid = ((rows + 16 * t.mf - 1) / (16 * t.mf)) * ((cols + tc - 1) / tc);
+        out->waves = r.waves;
+        out->tile_m = r.bm;
+        out->tile_n = out->item_width = r.tc;
+        out->items = out->grid = r.m_tiles * r.n_tiles;
+        if (r.kind == RowsPlan::kAlternating) out->grid = std::min(out->items, ws->cu_count);
         out->splits = 1;
         return QLIN_OK;
     }
@@ -1427,7 +1490,7 @@ int qlin_tune(qlin_workspace* ws, const qlin_weights* w, int32_t rows, uint32_t 
     const int path = fused ? 0 : (gemv_ok(ws, w, rows) ? 1 : 2);
     std::vector<int> cand;
     g_force_variant = -1;
-    if (!fused && pick_ks(ws, w, rows, w->Kp, flags) >= 0) cand.push_back(-1);
+    if (!fused && plan_rows(ws, w, rows, w->Kp, flags).kind != RowsPlan::kOther) cand.push_back(-1);
     g_force_variant = 0;
     const size_t own = cand.size();  // the planner's own choice comes first where it is not one of the variants
     if (path < 2) {

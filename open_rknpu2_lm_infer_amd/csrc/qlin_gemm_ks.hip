@@ -33,7 +33,7 @@
 //     512       14.7 (kept)     14.2 -> 11.0    32.2 (kept)          21.3 (kept)
 #include <hip/hip_fp16.h>
 
-#include "qlin_internal.hpp"
+#include "qlin_epilogue.hpp"
 
 namespace qlin {
 
@@ -226,8 +226,7 @@ __global__ __launch_bounds__(64 * WK) void gemm_ks_kernel(GemmParams p) {
     constexpr int NBO = SWIGLU ? NB / 2 : NB, TASKS = G::MFP * NBO;
     float* scl = reinterpret_cast<float*>(smem + G::SCL);
     if (tid < G::TM + G::TN) scl[tid] = pre;
-    const bool vec = (p.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(p.C) & 15) == 0;
-    const bool rvec = (p.ldr & 3) == 0 && (reinterpret_cast<uintptr_t>(p.R) & 15) == 0;
+    const bool vec = c_rows_vec(p), rvec = r_rows_vec(p);
 #pragma unroll
     for (int ph = 0; ph < MF / G::MFP; ++ph) {
         if (ph) lds_barrier();  // the previous fragments are read out
@@ -246,94 +245,19 @@ __global__ __launch_bounds__(64 * WK) void gemm_ks_kernel(GemmParams p) {
             const int m_in = (ph * G::MFP + rf) * 16 + lr;
             const int c_in = 16 * j + 4 * lc;
             const int m = m0 + m_in, c = n0 + c_in;
-            float res[4] = {0.0f, 0.0f, 0.0f, 0.0f};
             const bool live = m < p.M && c < ncols;
-            if (!SWIGLU && p.R && live) {
-                const int64_t at = (int64_t)m * p.ldr + c;
-                if (rvec && c + 3 < ncols) {
-                    if (p.r_f16) {
-                        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-                        const h4 v = *reinterpret_cast<const h4*>(reinterpret_cast<const _Float16*>(p.R) + at);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) res[e] = (float)v[e];
-                    } else {
-                        const float4 v = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(p.R) + at);
-                        res[0] = v.x; res[1] = v.y; res[2] = v.z; res[3] = v.w;
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (c + e < ncols)
-                            res[e] = p.r_f16 ? (float)reinterpret_cast<const _Float16*>(p.R)[at + e]
-                                             : reinterpret_cast<const float*>(p.R)[at + e];
-                }
-            }
-            v4i sg = {0, 0, 0, 0}, su = {0, 0, 0, 0};
+            float res[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (!SWIGLU && p.R && live) residual4(p, m, c, ncols, rvec, res);
+            v4i gate = {0, 0, 0, 0}, up = {0, 0, 0, 0};
 #pragma unroll
             for (int k = 0; k < WK; ++k) {
                 const uint8_t* at = smem + (((k * G::MFP + rf) * NB + j) << 10) + lane * 16;
-                sg += *reinterpret_cast<const v4i*>(at);
-                if constexpr (SWIGLU) su += *reinterpret_cast<const v4i*>(at + (NBO << 10));
+                gate += *reinterpret_cast<const v4i*>(at);
+                if constexpr (SWIGLU) up += *reinterpret_cast<const v4i*>(at + (NBO << 10));
             }
-            if (!live) continue;
-            const int64_t at = (int64_t)m * p.ldc + c;
-            if (p.c_kind == 2) {
-                int32_t* C = reinterpret_cast<int32_t*>(p.C) + at;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (BITS == 4) sg[e] >>= 4;
-                }
-                if (vec && c + 3 < ncols) {
-                    *reinterpret_cast<v4i*>(C) = sg;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (c + e < ncols) C[e] = sg[e];
-                }
-                continue;
-            }
-            const float sm = scl[m_in];
-            float o[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float gv = ((float)(BITS == 4 ? sg[e] >> 4 : sg[e]) * sm) * scl[G::TM + c_in + e];  // src/npu.rs:1117
-                if constexpr (SWIGLU) {
-                    const float uv = ((float)(BITS == 4 ? su[e] >> 4 : su[e]) * sm) * scl[G::TM + TC + c_in + e];
-                    o[e] = silu_gate(gv, uv);  // src/npu.rs:1202-1208
-                } else {
-                    o[e] = gv;
-                }
-            }
-            if (!SWIGLU && p.R) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {  // src/model/dense.rs:486-489
-                    const float y = o[e] * p.rmult;
-                    o[e] = res[e] + y;
-                }
-            }
-            if (p.c_kind == 1) {
-                _Float16* C = reinterpret_cast<_Float16*>(p.C) + at;
-                if (vec && c + 3 < ncols) {
-                    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-                    h4 v;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = f16_of_f32(o[e]);
-                    *reinterpret_cast<h4*>(C) = v;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (c + e < ncols) C[e] = f16_of_f32(o[e]);
-                }
-            } else {
-                float* C = reinterpret_cast<float*>(p.C) + at;
-                if (vec && c + 3 < ncols) {
-                    *reinterpret_cast<float4*>(C) = make_float4(o[0], o[1], o[2], o[3]);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (c + e < ncols) C[e] = o[e];
-                }
-            }
+            if (live)
+                finish4<BITS, SWIGLU>(p, p.c_kind, m, c, ncols, vec, gate, up, scl[m_in], scl + G::TM + c_in,
+                                      scl + G::TM + TC + c_in, res);
         }
     }
 }

@@ -147,6 +147,15 @@ constexpr int kKsConfigs = 20;
 KsTile gemm_ks_tile(int cfg);
 bool gemm_ks_fits(int bits, int cfg);  // two stages of every wave's ring fit the LDS
 hipError_t launch_gemm_ks(const GemmParams& p, int bits, int cfg, hipStream_t stream);
+// Tile of the alternating-waves GEMM: tokens x weight rows, what it is built for, its measured cost.
+struct PpTile {
+    int bm, bn;
+    bool w4, w8, plain, swiglu;
+    double step_us, step8_us, tile_us;
+};
+constexpr int kPpConfigs = 8;
+PpTile gemm_pp_tile(int cfg);
+hipError_t launch_gemm_pp(const GemmParams& p, int bits, int cfg, int cus, hipStream_t stream);
 hipError_t launch_swiglu(int rows, int F, const void* X, int x_f16, int64_t ldx, void* Y, int y_f16, int64_t ldy,
                          hipStream_t stream);
 hipError_t launch_pack_w4(const int8_t* codes_nk, int N, int K, int Np, int Kp, uint8_t* out,
