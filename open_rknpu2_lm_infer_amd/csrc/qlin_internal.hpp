@@ -44,6 +44,7 @@ struct QuantParams {
     int8_t* q;
     float* s;
     uint32_t* err;   // bit 0 set on non-finite input (may be null)
+    int err_on_host; // err is a word of pinned host memory, bit 0 its only use
     const float* gamma;  // RMSNorm weight, null = no norm
     float eps;
     uint32_t flags;

@@ -43,6 +43,14 @@ __device__ __forceinline__ void quant8(const float v[8], float inv, bool rne, bo
 }
 
 
+// Reports a row holding Inf / NaN.  A word in host memory gets a plain store: only bit 0 of it
+// is used, and an atomic on host memory would need the bus to carry it.
+__device__ __forceinline__ void flag_nonfinite(const QuantParams& p) {
+    if (!p.err) return;
+    if (p.err_on_host) __hip_atomic_store(p.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    else atomicOr(p.err, 1u);
+}
+
 template <typename T, bool VEC>
 __global__ __launch_bounds__(kRowThreads) void quant_rows_kernel(QuantParams p) {
     __shared__ float lds[8];
@@ -77,7 +85,7 @@ __global__ __launch_bounds__(kRowThreads) void quant_rows_kernel(QuantParams p) 
     }
     if (threadIdx.x == 0) {
         p.s[row] = s;
-        if (bad && p.err) atomicOr(p.err, 1u);
+        if (bad) flag_nonfinite(p);
     }
 }
 
@@ -198,7 +206,7 @@ __global__ __launch_bounds__(NT) void quant_rows_staged_kernel(QuantParams p) {
     }
     if (t == 0) {
         p.s[row] = s;
-        if (f && p.err) atomicOr(p.err, 1u);
+        if (f) flag_nonfinite(p);
     }
 }
 
@@ -350,7 +358,7 @@ __global__ __launch_bounds__(1024) void quant_norm_block_kernel(QuantParams p) {
     for (int k0 = p.K + 8 * t; k0 < p.ldq; k0 += 8 * nt) *reinterpret_cast<uint2*>(qrow + k0) = make_uint2(0, 0);
     if (t == 0) {
         p.s[row] = s;
-        if (f && p.err) atomicOr(p.err, 1u);
+        if (f) flag_nonfinite(p);
     }
 }
 
@@ -452,7 +460,7 @@ __global__ __launch_bounds__(64) void quant_norm_wave_kernel(QuantParams p) {
     for (int k0 = p.K + 8 * lane; k0 < p.ldq; k0 += 8 * 64) *reinterpret_cast<uint2*>(qrow + k0) = make_uint2(0, 0);
     if (lane == 0) {
         p.s[row] = s;
-        if (f && p.err) atomicOr(p.err, 1u);
+        if (f) flag_nonfinite(p);
     }
 }
 
@@ -574,7 +582,7 @@ __global__ __launch_bounds__(256) void quant_rows_reg_kernel(QuantParams p, int 
     for (int k0 = p.K + 8 * lane; k0 < p.ldq; k0 += 8 * L) *reinterpret_cast<uint2*>(qrow + k0) = make_uint2(0, 0);
     if (lane == 0) {
         p.s[row] = s;
-        if (bad && p.err) atomicOr(p.err, 1u);
+        if (bad) flag_nonfinite(p);
     }
 }
 
