@@ -62,7 +62,7 @@ struct qlin_workspace {
     hipStream_t last;    // stream of the most recent run
     uint64_t device_bytes;
     bool counted;        // among the workspaces that keep staging sets alive
-    bool async_used;     // a run other than the host-buffer ones may have set err
+    bool err_used;       // a run that reports in err itself may have set it (also by a later graph replay)
 };
 
 namespace {
@@ -113,11 +113,15 @@ HostStage* take_stage(int device) {
     if (!h) return nullptr;
     h->device = device;
     void *m = nullptr, *d = nullptr;
+    // another thread may be capturing a graph, which an allocation would end otherwise
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
     bool ok = hipHostMalloc(&m, 2 * kSlots * kSlotBytes + 256, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess;
     h->mem = static_cast<uint8_t*>(m);
     ok = ok && hipHostGetDevicePointer(&d, m, 0) == hipSuccess;
     h->dev = static_cast<uint8_t*>(d);
     for (int i = 0; ok && i < kSlots; ++i) ok = hipEventCreateWithFlags(&h->done[i], hipEventDisableTiming) == hipSuccess;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (!ok) {
         free_stage(h);
         return nullptr;
@@ -1068,7 +1072,7 @@ int run_impl(qlin_workspace* ws, const qlin_weights* w, int rows, const void* A,
     if (ldc < ncols) return QLIN_ERR_PARAM;
     if (gamma && !(eps > 0.0f && std::isfinite(eps))) return QLIN_ERR_PARAM;
     ws->last = st;
-    ws->async_used = true;
+    ws->err_used = true;
     if (gemv_fusable(ws, w, rows, A, lda, gamma, flags)) {
         return run_gemv(ws, w, rows, A, a_dtype == QLIN_F16, lda, gamma, eps, nullptr, 0, nullptr, C,
                         c_dtype == QLIN_F16, ldc, flags, st, res);
@@ -1093,6 +1097,7 @@ int run_impl(qlin_workspace* ws, const qlin_weights* w, int rows, const void* A,
 int run_host_copies(qlin_workspace* ws, const qlin_weights* w, int rows, const float* A, float* C, int ncols,
                     uint32_t flags) {
     hipStream_t st = ws->stream;
+    ws->err_used = true;
     if (hipMemsetAsync(ws->err, 0, sizeof(uint32_t), st) != hipSuccess) return QLIN_ERR_DEVICE;
     if (hipMemcpyAsync(ws->dA, A, (size_t)rows * w->K * sizeof(float), hipMemcpyHostToDevice, st) != hipSuccess)
         return QLIN_ERR_DEVICE;
@@ -1124,8 +1129,14 @@ int run_host(qlin_workspace* ws, const qlin_weights* w, int rows, const float* A
     const int ncols = (flags & kFlagSwiglu) ? w->N / 2 : w->N;
     const size_t row_in = (size_t)w->K * sizeof(float), row_out = (size_t)ncols * sizeof(float);
     const size_t per_slot = kSlotBytes / std::max(row_in, row_out);
-    // rows whose quantization would read them by elements, or longer than a slot
-    if (w->K % 8 || per_slot == 0) return run_host_copies(ws, w, rows, A, C, ncols, flags);
+    // rows whose quantization would read them by elements, or longer than a slot; buffers that
+    // overlap, where a block's rows out could land on rows that are still to go in; a thread on
+    // another device, whose events this stream could not record
+    const uintptr_t a0 = reinterpret_cast<uintptr_t>(A), c0 = reinterpret_cast<uintptr_t>(C);
+    const bool overlap = a0 < c0 + (size_t)rows * row_out && c0 < a0 + (size_t)rows * row_in;
+    int device = -1;
+    if (w->K % 8 || per_slot == 0 || overlap || hipGetDevice(&device) != hipSuccess || device != ws->device)
+        return run_host_copies(ws, w, rows, A, C, ncols, flags);
     HostStage* h = take_stage(ws->device);
     if (!h) return run_host_copies(ws, w, rows, A, C, ncols, flags);
     hipStream_t st = ws->stream;
@@ -1135,7 +1146,7 @@ int run_host(qlin_workspace* ws, const qlin_weights* w, int rows, const float* A
     const int blocks = (int)((rows + per_slot - 1) / per_slot), step = (rows + blocks - 1) / blocks;
     int rc = QLIN_OK;
     // the workspace's word reports this call, as every host-buffer call's
-    if (ws->async_used && hipMemsetAsync(ws->err, 0, sizeof(uint32_t), st) != hipSuccess) rc = QLIN_ERR_DEVICE;
+    if (ws->err_used && hipMemsetAsync(ws->err, 0, sizeof(uint32_t), st) != hipSuccess) rc = QLIN_ERR_DEVICE;
     auto rows_of = [&](int b) { return std::min(step, rows - b * step); };
     auto finish = [&](int b) {  // waits for block b and copies its rows out
         if (!rc && hipEventSynchronize(h->done[b % kSlots]) != hipSuccess) rc = QLIN_ERR_DEVICE;
@@ -1169,9 +1180,10 @@ int run_host(qlin_workspace* ws, const qlin_weights* w, int rows, const float* A
         (void)hipStreamSynchronize(st);  // nothing still uses the set
     } else if (*const_cast<volatile uint32_t*>(err_host)) {
         rc = QLIN_ERR_NONFINITE;
-        const uint32_t one = 1;
-        if (hipMemcpy(ws->err, &one, sizeof(one), hipMemcpyHostToDevice) != hipSuccess) rc = QLIN_ERR_DEVICE;
-        ws->async_used = true;  // so that the next call clears it
+        ws->err_used = true;  // so that the next call clears it
+        if (hipMemcpyAsync(ws->err, err_host, sizeof(uint32_t), hipMemcpyHostToDevice, st) != hipSuccess ||
+            hipStreamSynchronize(st) != hipSuccess)
+            rc = QLIN_ERR_DEVICE;
     }
     give_back_stage(h);
     return rc;

@@ -2,12 +2,14 @@
 against the device entry point bit for bit at one block, several blocks (more than the slots)
 and a ragged last one, at the forms that go through plain copies (K not a multiple of 8, rows
 longer than a slot); the error word of a call and of the workspace; several threads at once."""
+import ctypes
 import threading
 
 import numpy as np
 import pytest
 import torch
 
+from open_rknpu2_lm_infer_amd import _lib
 from open_rknpu2_lm_infer_amd import qlinear as ql
 from open_rknpu2_lm_infer_amd import synth
 from open_rknpu2_lm_infer_amd._lib import QLIN_ERR_NONFINITE, QLIN_OK, QlinError
@@ -60,6 +62,37 @@ def test_host_run_error_word():
     ql.run(ws, w, x)
     torch.cuda.synchronize()
     assert np.array_equal(ql.run_host_f32(ws, w, A), ref) and ws.status(clear=False) == QLIN_OK
+    ws.close()
+    w.close()
+
+
+def test_host_run_clears_the_word_of_a_run_through_copies():
+    """A call whose rows go through plain copies (K = 1002) sets the workspace's word itself; the
+    next call through the slots starts clean."""
+    w, wide = weights(4, 2560, 256, 975), weights(4, 1002, 256, 976)
+    ws = ql.Workspace(4, 2560, 256)
+    bad = synth.activations(4, 1002, 977).float().numpy()
+    bad[2, 5] = np.inf
+    with pytest.raises(QlinError):
+        ql.run_host_f32(ws, wide, bad)
+    assert ws.status(clear=False) == QLIN_ERR_NONFINITE
+    ql.run_host_f32(ws, w, synth.activations(4, 2560, 978).float().numpy())
+    assert ws.status(clear=False) == QLIN_OK
+    for x in (ws, w, wide):
+        x.close()
+
+
+def test_host_run_over_its_own_input():
+    """C at A, with rows out longer than rows in, over several blocks: every row is read first."""
+    K, N, rows = 1024, 2048, 500
+    w, ws = weights(8, K, N, 985), ql.Workspace(rows, K, N)
+    A = synth.activations(rows, K, 986).float().numpy()
+    want = ql.run_host_f32(ws, w, A)
+    buf = np.zeros(rows * N, np.float32)
+    buf[:rows * K] = A.reshape(-1)
+    at = buf.ctypes.data_as(ctypes.c_void_p)
+    assert _lib.load().qlin_run_f32(ws.handle, w.handle, rows, at, at) == QLIN_OK
+    assert np.array_equal(buf.reshape(rows, N), want)
     ws.close()
     w.close()
 
