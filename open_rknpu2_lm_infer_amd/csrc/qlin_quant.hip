@@ -210,14 +210,6 @@ __global__ __launch_bounds__(NT) void quant_rows_staged_kernel(QuantParams p) {
     }
 }
 
-// RMSNorm rows, one wave per row, row and RMSNorm weights in registers: the lane's NC
-// 16-byte row chunks and their weights are all loaded before any is used, the row is
-// copied into LDS only for the norm sum (the reference's chain order reads it there),
-// and the normalized values stay in registers for the absmax and the quantize pass.
-// The staged kernel loads the weights again in both passes, a dependent global round
-// trip per 8 values (M = 4096, K = 2560: 17.5 us there).  Same arithmetic as the staged
-// kernel, value for value.  Needs K % 8 == 0, a 16-byte aligned row and weights, an
-// 8-byte aligned q with ldq % 8 == 0, and 64 * NC chunks >= K / E.
 // Sum of squares in the order of src/model/cpu.rs:14-35 (16 fused-multiply-add chains,
 // chain j takes elements j, j+16, ... in order, combined lanewise as (a+b)+(c+d), then
 // (t0+t1)+(t2+t3); K % 16 == 0 so there is no scalar tail), from a row stored
@@ -375,6 +367,14 @@ static bool launch_quant_block(const QuantParams& p, int rows, hipStream_t strea
     return true;
 }
 
+// RMSNorm rows, one wave per row, row and RMSNorm weights in registers: the lane's NC
+// 16-byte row chunks and their weights are all loaded before any is used, the row is
+// copied into LDS only for the norm sum (the reference's chain order reads it there),
+// and the normalized values stay in registers for the absmax and the quantize pass.
+// The staged kernel loads the weights again in both passes, a dependent global round
+// trip per 8 values (M = 4096, K = 2560: 17.5 us there).  Same arithmetic as the staged
+// kernel, value for value.  Needs K % 8 == 0, a 16-byte aligned row and weights, an
+// 8-byte aligned q with ldq % 8 == 0, and 64 * NC chunks >= K / E.
 template <typename T, int NC, bool CM>
 __global__ __launch_bounds__(64) void quant_norm_wave_kernel(QuantParams p) {
     extern __shared__ __align__(16) uint8_t stage[];
