@@ -912,11 +912,11 @@ RowsPlan rows_tiles(RowsPlan::Kind kind, int cfg, int bm, int bn, int waves, con
 
 // Where the wave-split-K estimate is too low, over 6084 random shapes (K 384..9728, N 256..19456,
 // 9..4096 rows, both kernels timed): large tiles over a K of at most six steps, whose epilogue is
-// most of the launch (68 shapes, the others in 0.96 of its time; W4 K =
+// most of the launch (68 shapes, the others in 0.96 of its geometric mean; W4 K =
 // 512, N = 7680, 167 rows 7.7 -> 6.5 us); W8 tiles of 96 channels over 36 steps and more (15
 // shapes, 0.91; K = 8576, N = 2944, 219 rows 30.3 -> 18.3); and tiles of 64 and more rows over as
 // many steps above 1792 rows, where every workgroup of a row block streams the same long rows (0.91;
-// W8 K = 6400, N = 384, 2728 rows 26.5 -> 18.1).  Elsewhere it took 0.4..0.9 of the others' time.
+// W8 K = 6400, N = 384, 2728 rows 26.5 -> 18.1).  By tile height and K it takes 0.4..1.0 elsewhere.
 bool gemm_ks_lags(const KsTile& t, int steps, int rows, bool w4) {
     if (steps <= 6) return t.mf * t.nb >= (w4 ? 20 : 18);
     return steps >= 36 && ((!w4 && t.nb == 6) || (t.mf >= 4 && rows > 1792));
