@@ -1,7 +1,7 @@
 """Builds libqlinear.so and libqlinear.a (the HIP kernels, the C ABI and the C++ npu
 mirror) in-tree for gfx950, libqlcalib.so (the calibration kernels of bench.py --mode
 calib, not part of the library), and the native test binaries under tests/cpp/_build:
-the npu mirror's test and a C program linked against the static archive.
+the npu mirror's test, the host-call test and a C program linked against the static archive.
 
     python -m open_rknpu2_lm_infer_amd.build
 
@@ -52,6 +52,8 @@ ROOT = os.path.dirname(HERE)
 TEST_SRC = os.path.join(ROOT, "tests", "cpp", "npu_backend_test.cpp")
 TEST_BUILD = os.path.join(ROOT, "tests", "cpp", "_build")
 TEST_BIN = os.path.join(TEST_BUILD, "npu_backend_test")
+HOST_TEST_SRC = os.path.join(ROOT, "tests", "cpp", "host_calls_test.cpp")
+HOST_TEST_BIN = os.path.join(TEST_BUILD, "host_calls_test")
 STATIC_TEST_SRC = os.path.join(ROOT, "tests", "cpp", "static_link_test.c")
 STATIC_TEST_BIN = os.path.join(TEST_BUILD, "static_link_test")
 
@@ -111,13 +113,18 @@ def build_calib() -> str:
 
 
 def build_tests() -> str:
-    """Native test of the npu mirror; its checker (the CPU oracle) is compiled in."""
+    """Native tests: the npu mirror (its checker, the CPU oracle, is compiled in), the host side
+    of the host-buffer calls and the static archive."""
     os.makedirs(TEST_BUILD, exist_ok=True)
     oracle_obj = os.path.join(TEST_BUILD, "qlin_oracle.o")
     subprocess.run(["gcc", "-O2", "-fPIC", "-ffp-contract=off", "-fno-fast-math", "-std=c11", "-c",
                     os.path.join(ROOT, "oracle", "qlin_oracle.c"), "-o", oracle_obj], check=True)
     subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", TEST_SRC, oracle_obj, "-o", TEST_BIN,
                     f"-L{HERE}", "-lqlinear", "-Wl,-rpath,$ORIGIN/../../../open_rknpu2_lm_infer_amd", "-lm"], check=True)
+    # its own definitions of the HIP calls take the place of the runtime's
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", HOST_TEST_SRC, "-o",
+                    HOST_TEST_BIN, "-rdynamic", f"-L{HERE}", "-lqlinear",
+                    "-Wl,-rpath,$ORIGIN/../../../open_rknpu2_lm_infer_amd"], check=True)
     # a C caller of the static archive, linked as a Rust build.rs would link it (its GPU
     # mode checks the kernels against the oracle, compiled in as the checker)
     static_obj = os.path.join(TEST_BUILD, "static_link_test.o")

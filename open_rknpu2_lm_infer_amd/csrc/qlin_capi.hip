@@ -75,7 +75,7 @@ namespace {
 // so calls on several threads and streams use different sets.
 constexpr int kSlots = 4;
 constexpr size_t kSlotBytes = (size_t)1 << 20;  // of rows in and of rows out
-constexpr size_t kIdleSets = 4;
+constexpr int kIdleSets = 4;
 
 struct HostStage {
     int device;
@@ -84,12 +84,16 @@ struct HostStage {
     hipEvent_t done[kSlots];
 };
 
-std::mutex g_stage_mutex;
-std::vector<HostStage*>& idle_stages() {
-    static std::vector<HostStage*> v;
-    return v;
+// Never destroyed (no destructor runs for any of these): the owner of a workspace may be an
+// object with static storage, whose destructor comes after those of whatever this file built
+// while the program ran.
+std::mutex& stage_mutex() {
+    static std::mutex& m = *new std::mutex;
+    return m;
 }
-int g_workspaces = 0;  // live ones, under g_stage_mutex
+HostStage* g_idle[kIdleSets];  // idle sets, under stage_mutex as the counts
+int g_n_idle = 0;
+int g_workspaces = 0;          // live workspaces
 
 void free_stage(HostStage* h) {
     for (hipEvent_t e : h->done)
@@ -100,12 +104,11 @@ void free_stage(HostStage* h) {
 
 HostStage* take_stage(int device) {
     {
-        std::lock_guard<std::mutex> g(g_stage_mutex);
-        auto& v = idle_stages();
-        for (size_t i = 0; i < v.size(); ++i)
-            if (v[i]->device == device) {
-                HostStage* h = v[i];
-                v.erase(v.begin() + (long)i);
+        std::lock_guard<std::mutex> g(stage_mutex());
+        for (int i = 0; i < g_n_idle; ++i)
+            if (g_idle[i]->device == device) {
+                HostStage* h = g_idle[i];
+                g_idle[i] = g_idle[--g_n_idle];
                 return h;
             }
     }
@@ -131,9 +134,9 @@ HostStage* take_stage(int device) {
 
 void give_back_stage(HostStage* h) {
     {
-        std::lock_guard<std::mutex> g(g_stage_mutex);
-        if (g_workspaces > 0 && idle_stages().size() < kIdleSets) {
-            idle_stages().push_back(h);
+        std::lock_guard<std::mutex> g(stage_mutex());
+        if (g_workspaces > 0 && g_n_idle < kIdleSets) {
+            g_idle[g_n_idle++] = h;
             return;
         }
     }
@@ -142,13 +145,14 @@ void give_back_stage(HostStage* h) {
 
 // Counts a workspace in (+1) or out (-1); the last one out frees the idle sets.
 void count_workspace(int d) {
-    std::vector<HostStage*> drop;
+    HostStage* drop[kIdleSets];
+    int n = 0;
     {
-        std::lock_guard<std::mutex> g(g_stage_mutex);
+        std::lock_guard<std::mutex> g(stage_mutex());
         g_workspaces += d;
-        if (g_workspaces == 0) drop.swap(idle_stages());
+        while (g_workspaces == 0 && g_n_idle > 0) drop[n++] = g_idle[--g_n_idle];
     }
-    for (HostStage* h : drop) free_stage(h);
+    while (n > 0) free_stage(drop[--n]);
 }
 
 }  // namespace

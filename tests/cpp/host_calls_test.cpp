@@ -1,0 +1,134 @@
+// Host side of the host-buffer entry points without a GPU: the HIP calls of libqlinear.so
+// bind to the definitions below (device memory is host memory, kernels do not run), so what
+// is checked is the library's own bookkeeping.
+//
+//   host_calls_test exit        a workspace owned by an object with static storage, used by a
+//                               host-buffer call, is freed after main returns
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <string>
+#include <vector>
+
+#include <hip/hip_runtime_api.h>
+
+#include "../../include/qlinear.h"
+
+#ifdef hipGetDeviceProperties
+#undef hipGetDeviceProperties
+#endif
+
+namespace {
+hipError_t g_last = hipSuccess;  // as the runtime keeps it: until it is read
+hipError_t err(hipError_t e) {
+    if (e != hipSuccess) g_last = e;
+    return e;
+}
+hipError_t alloc(void** p, size_t n) {
+    *p = std::calloc(1, n ? n : 1);
+    return err(*p ? hipSuccess : hipErrorOutOfMemory);
+}
+}  // namespace
+
+extern "C" {
+hipError_t hipGetLastError() {
+    const hipError_t e = g_last;
+    g_last = hipSuccess;
+    return e;
+}
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipMalloc(void** p, size_t n) { return alloc(p, n); }
+hipError_t hipFree(void* p) { return std::free(p), hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return alloc(p, n); }
+hipError_t hipHostFree(void* p) { return std::free(p), hipSuccess; }
+hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) { return *d = h, hipSuccess; }
+hipError_t hipMemset(void* p, int v, size_t n) { return std::memset(p, v, n), hipSuccess; }
+hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) { return std::memset(p, v, n), hipSuccess; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+    return std::memcpy(d, s, n), hipSuccess;
+}
+hipError_t hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, hipMemcpyKind, hipStream_t) {
+    for (size_t i = 0; i < h; ++i) std::memcpy(static_cast<char*>(d) + i * dp, static_cast<const char*>(s) + i * sp, w);
+    return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+    void* p;
+    const hipError_t e = alloc(&p, 1);
+    *s = static_cast<hipStream_t>(p);
+    return e;
+}
+hipError_t hipStreamDestroy(hipStream_t s) { return std::free(s), hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    void* p;
+    const hipError_t r = alloc(&p, 1);
+    *e = static_cast<hipEvent_t>(p);
+    return r;
+}
+hipError_t hipEventDestroy(hipEvent_t e) { return std::free(e), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
+    static thread_local hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;
+    const hipStreamCaptureMode was = mode;
+    mode = *m;
+    *m = was;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) { return hipSuccess; }
+}
+
+namespace {
+
+// A linear and its workspace.
+struct Pair {
+    qlin_weights* w = nullptr;
+    qlin_workspace* ws = nullptr;
+    int K = 0, N = 0;
+    int open(int bits, int k, int n, int rows) {
+        K = k;
+        N = n;
+        const qlin_weight_config cfg = {bits, K, N};
+        const std::vector<int8_t> packed((size_t)N * K * bits / 8);
+        const std::vector<float> scales(N, 1.0f);
+        if (int rc = qlin_weights_create_packed(&cfg, packed.data(), scales.data(), &w)) return rc;
+        return qlin_workspace_create(rows, K, N, &ws);
+    }
+    int run(int rows) {
+        const std::vector<float> a((size_t)rows * K, 0.5f);
+        std::vector<float> c((size_t)rows * N);
+        return qlin_run_f32(ws, w, rows, a.data(), c.data());
+    }
+    ~Pair() {
+        qlin_workspace_free(ws);
+        qlin_weights_free(w);
+    }
+};
+
+Pair g_owner;  // freed after main, and after everything the library builds during main
+
+int expect(bool ok, const char* what) {
+    if (!ok) std::printf("FAIL %s\n", what);
+    return ok ? 0 : 1;
+}
+
+int at_exit() {
+    if (expect(g_owner.open(4, 256, 256, 4) == QLIN_OK, "create")) return 1;
+    return expect(g_owner.run(4) == QLIN_OK, "run");
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const std::string mode = argc > 1 ? argv[1] : "";
+    const int rc = mode == "exit" ? at_exit() : expect(false, "mode");
+    if (!rc) std::printf("PASS %s\n", mode.c_str());
+    std::fflush(stdout);
+    return rc;
+}
