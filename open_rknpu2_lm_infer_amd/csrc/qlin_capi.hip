@@ -127,6 +127,7 @@ HostStage* take_stage(int device) {
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (!ok) {
         free_stage(h);
+        (void)hipGetLastError();  // kept by the runtime until it is read: a launch would be taken to have failed
         return nullptr;
     }
     return h;

@@ -4,6 +4,8 @@
 //
 //   host_calls_test exit        a workspace owned by an object with static storage, used by a
 //                               host-buffer call, is freed after main returns
+//   host_calls_test no_pinned   pinned memory runs out: the rows go through plain copies, and
+//                               the failed calls' error is not taken for a launch's
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -30,6 +32,9 @@ hipError_t alloc(void** p, size_t n) {
     *p = std::calloc(1, n ? n : 1);
     return err(*p ? hipSuccess : hipErrorOutOfMemory);
 }
+enum Fail { kNone, kHostMalloc, kHostPointer, kEvent };
+Fail g_fail = kNone;  // the call that fails
+int g_copied_in = 0;  // rows or words copied to device memory
 }  // namespace
 
 extern "C" {
@@ -43,13 +48,18 @@ hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v 
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipMalloc(void** p, size_t n) { return alloc(p, n); }
 hipError_t hipFree(void* p) { return std::free(p), hipSuccess; }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return alloc(p, n); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    return g_fail == kHostMalloc ? err(hipErrorOutOfMemory) : alloc(p, n);
+}
 hipError_t hipHostFree(void* p) { return std::free(p), hipSuccess; }
-hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) { return *d = h, hipSuccess; }
+hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) {
+    return *d = h, g_fail == kHostPointer ? err(hipErrorInvalidValue) : hipSuccess;
+}
 hipError_t hipMemset(void* p, int v, size_t n) { return std::memset(p, v, n), hipSuccess; }
 hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) { return std::memset(p, v, n), hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) {
+    g_copied_in += k == hipMemcpyHostToDevice;
     return std::memcpy(d, s, n), hipSuccess;
 }
 hipError_t hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, hipMemcpyKind, hipStream_t) {
@@ -65,8 +75,8 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
 hipError_t hipStreamDestroy(hipStream_t s) { return std::free(s), hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
-    void* p;
-    const hipError_t r = alloc(&p, 1);
+    void* p = nullptr;
+    const hipError_t r = g_fail == kEvent ? err(hipErrorOutOfMemory) : alloc(&p, 1);
     *e = static_cast<hipEvent_t>(p);
     return r;
 }
@@ -123,11 +133,29 @@ int at_exit() {
     return expect(g_owner.run(4) == QLIN_OK, "run");
 }
 
+int no_pinned() {
+    int bad = 0;
+    for (Fail f : {kHostMalloc, kHostPointer, kEvent}) {
+        Pair p;
+        if (expect(p.open(4, 256, 256, 4) == QLIN_OK, "create")) return 1;
+        for (int call = 0; call < 2; ++call) {
+            g_fail = f;
+            g_copied_in = 0;
+            bad |= expect(p.run(4) == QLIN_OK, "run through copies") | expect(g_copied_in == 1, "rows copied");
+            g_fail = kNone;
+            bad |= expect(hipGetLastError() == hipSuccess, "no error left behind");
+        }
+        g_copied_in = 0;  // and once it is there again, through the pinned blocks
+        bad |= expect(p.run(4) == QLIN_OK, "run") | expect(g_copied_in == 0, "rows through pinned blocks");
+    }
+    return bad;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::string mode = argc > 1 ? argv[1] : "";
-    const int rc = mode == "exit" ? at_exit() : expect(false, "mode");
+    const int rc = mode == "exit" ? at_exit() : mode == "no_pinned" ? no_pinned() : expect(false, "mode");
     if (!rc) std::printf("PASS %s\n", mode.c_str());
     std::fflush(stdout);
     return rc;
