@@ -158,7 +158,9 @@ int qlin_workspace_status(qlin_workspace* ws, int32_t clear);
 /* ---- host-buffer runs: the drop-in for the reference's synchronous calls ----
  * Replaces rk_npu_w4a8_run_f32 (src/npu.rs:1047-1049) and rk_npu_f32i8f32_run_dynamic
  * (src/npu.rs:1052-1061): A f32 [rows, K] and C f32 [rows, N] are host pointers;
- * the call returns after C is written.  Non-finite input returns QLIN_ERR_NONFINITE. */
+ * the call returns after C is written.  Non-finite input returns QLIN_ERR_NONFINITE.  The call
+ * waits for the GPU, so no graph can be captured around it: other threads may record one beside it
+ * in the thread-local or relaxed capture mode, but not in the global one. */
 int qlin_run_f32(qlin_workspace* ws, const qlin_weights* weights, int32_t rows, const float* A,
                  float* C);
 

@@ -123,7 +123,7 @@ def build_tests() -> str:
                     f"-L{HERE}", "-lqlinear", "-Wl,-rpath,$ORIGIN/../../../open_rknpu2_lm_infer_amd", "-lm"], check=True)
     # its own definitions of the HIP calls take the place of the runtime's
     subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", HOST_TEST_SRC, "-o",
-                    HOST_TEST_BIN, "-rdynamic", f"-L{HERE}", "-lqlinear",
+                    HOST_TEST_BIN, "-rdynamic", "-pthread", f"-L{HERE}", "-lqlinear",
                     "-Wl,-rpath,$ORIGIN/../../../open_rknpu2_lm_infer_amd"], check=True)
     # a C caller of the static archive, linked as a Rust build.rs would link it (its GPU
     # mode checks the kernels against the oracle, compiled in as the checker)

@@ -95,7 +95,16 @@ HostStage* g_idle[kIdleSets];  // idle sets, under stage_mutex as the counts
 int g_n_idle = 0;
 int g_workspaces = 0;          // live workspaces
 
+// Keeps allocations and frees out of the checks of a graph that another thread records in global
+// capture mode.  (The copies and waits of a host-buffer call end such a capture all the same.)
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 void free_stage(HostStage* h) {
+    const RelaxedCapture relaxed;
     for (hipEvent_t e : h->done)
         if (e) (void)hipEventDestroy(e);
     if (h->mem) (void)hipHostFree(h->mem);
@@ -116,15 +125,12 @@ HostStage* take_stage(int device) {
     if (!h) return nullptr;
     h->device = device;
     void *m = nullptr, *d = nullptr;
-    // another thread may be capturing a graph, which an allocation would end otherwise
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const RelaxedCapture relaxed;
     bool ok = hipHostMalloc(&m, 2 * kSlots * kSlotBytes + 256, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess;
     h->mem = static_cast<uint8_t*>(m);
     ok = ok && hipHostGetDevicePointer(&d, m, 0) == hipSuccess;
     h->dev = static_cast<uint8_t*>(d);
     for (int i = 0; ok && i < kSlots; ++i) ok = hipEventCreateWithFlags(&h->done[i], hipEventDisableTiming) == hipSuccess;
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (!ok) {
         free_stage(h);
         (void)hipGetLastError();  // kept by the runtime until it is read: a launch would be taken to have failed

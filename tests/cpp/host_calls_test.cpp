@@ -6,12 +6,15 @@
 //                               host-buffer call, is freed after main returns
 //   host_calls_test no_pinned   pinned memory runs out: the rows go through plain copies, and
 //                               the failed calls' error is not taken for a launch's
+//   host_calls_test capture     sets are allocated and freed in the relaxed capture mode, also
+//                               the set of a call beyond those that stay idle
+#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include <hip/hip_runtime_api.h>
@@ -23,7 +26,18 @@
 #endif
 
 namespace {
-hipError_t g_last = hipSuccess;  // as the runtime keeps it: until it is read
+thread_local hipError_t g_last = hipSuccess;  // as the runtime keeps it: until it is read
+thread_local hipStreamCaptureMode g_mode = hipStreamCaptureModeGlobal;
+std::mutex g_mutex;
+int g_pinned = 0, g_events = 0;  // live allocations, under g_mutex
+bool g_exposed = false;          // one was made or freed outside the relaxed capture mode
+int g_gate = 0;                  // event waits still to come before any returns
+std::condition_variable g_gate_open;
+void count(int& what, int d) {
+    std::lock_guard<std::mutex> g(g_mutex);
+    what += d;
+    g_exposed |= g_mode != hipStreamCaptureModeRelaxed;
+}
 hipError_t err(hipError_t e) {
     if (e != hipSuccess) g_last = e;
     return e;
@@ -49,9 +63,14 @@ hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipMalloc(void** p, size_t n) { return alloc(p, n); }
 hipError_t hipFree(void* p) { return std::free(p), hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
-    return g_fail == kHostMalloc ? err(hipErrorOutOfMemory) : alloc(p, n);
+    if (g_fail == kHostMalloc) return err(hipErrorOutOfMemory);
+    count(g_pinned, 1);
+    return alloc(p, n);
 }
-hipError_t hipHostFree(void* p) { return std::free(p), hipSuccess; }
+hipError_t hipHostFree(void* p) {
+    count(g_pinned, -1);
+    return std::free(p), hipSuccess;
+}
 hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) {
     return *d = h, g_fail == kHostPointer ? err(hipErrorInvalidValue) : hipSuccess;
 }
@@ -77,17 +96,25 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
     void* p = nullptr;
     const hipError_t r = g_fail == kEvent ? err(hipErrorOutOfMemory) : alloc(&p, 1);
+    if (p) count(g_events, 1);
     *e = static_cast<hipEvent_t>(p);
     return r;
 }
-hipError_t hipEventDestroy(hipEvent_t e) { return std::free(e), hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) {
+    count(g_events, -1);
+    return std::free(e), hipSuccess;
+}
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) {
+    std::unique_lock<std::mutex> g(g_mutex);
+    if (g_gate > 0 && --g_gate == 0) g_gate_open.notify_all();
+    g_gate_open.wait(g, [] { return g_gate == 0; });
+    return hipSuccess;
+}
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
-    static thread_local hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;
-    const hipStreamCaptureMode was = mode;
-    mode = *m;
+    const hipStreamCaptureMode was = g_mode;
+    g_mode = *m;
     *m = was;
     return hipSuccess;
 }
@@ -151,11 +178,30 @@ int no_pinned() {
     return bad;
 }
 
+int capture() {
+    constexpr int kCalls = 6, kIdle = 4;
+    int bad = 0;
+    {
+        Pair p[kCalls];
+        for (Pair& x : p)
+            if (expect(x.open(4, 256, 256, 4) == QLIN_OK, "create")) return 1;
+        g_gate = kCalls;  // every call holds a set of its own before any gives it back
+        std::vector<std::thread> threads;
+        for (Pair& x : p) threads.emplace_back([&bad, &x] {
+            if (x.run(4) != QLIN_OK) bad = 1;
+        });
+        for (std::thread& t : threads) t.join();
+        bad |= expect(!bad, "runs") | expect(g_pinned == kIdle, "sets kept") | expect(!g_exposed, "sets given back");
+    }
+    return bad | expect(g_pinned == 0 && g_events == 0, "nothing kept without a workspace") |
+           expect(!g_exposed, "sets freed with the last workspace");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::string mode = argc > 1 ? argv[1] : "";
-    const int rc = mode == "exit" ? at_exit() : mode == "no_pinned" ? no_pinned() : expect(false, "mode");
+    const int rc = mode == "exit" ? at_exit() : mode == "no_pinned" ? no_pinned() : mode == "capture" ? capture() : expect(false, "mode");
     if (!rc) std::printf("PASS %s\n", mode.c_str());
     std::fflush(stdout);
     return rc;

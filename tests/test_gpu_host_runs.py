@@ -97,6 +97,42 @@ def test_host_run_over_its_own_input():
     w.close()
 
 
+@pytest.mark.parametrize("mode", ["thread_local", "relaxed"])
+def test_host_runs_beside_a_capture(mode):
+    """Six host-buffer calls on threads of their own, more than the idle sets kept (so that sets
+    are allocated and freed), while this thread records a graph: both give their usual results."""
+    K, N = 2560, 2560
+    w = weights(4, K, N, 987)
+    x, y = synth.activations(64, K, 988).to(DEV), torch.empty((64, N), dtype=torch.float16, device=DEV)
+    ws, spaces = ql.Workspace(64, K, N), [ql.Workspace(30, K, N) for _ in range(6)]
+    rows = synth.activations(30, K, 989).float().numpy()
+    want = ql.run(ws, w, x).clone()
+    host = ql.run(spaces[0], w, torch.from_numpy(rows).to(DEV), out_dtype=torch.float32).cpu().numpy()
+    torch.cuda.synchronize()
+    got, meet = [], threading.Barrier(6)
+
+    def work(space):
+        meet.wait()
+        got.append(ql.run_host_f32(space, w, rows))
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in spaces]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, capture_error_mode=mode):
+        ql.run(ws, w, x, out=y)
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    assert len(got) == 6 and all(np.array_equal(o, host) for o in got)
+    for _ in range(2):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+    for s in (ws, *spaces, w):
+        s.close()
+
+
 def test_host_runs_on_several_threads():
     """Six threads, a workspace each, more than the idle sets kept: every call gets its own rows."""
     K, N = 2560, 2560
