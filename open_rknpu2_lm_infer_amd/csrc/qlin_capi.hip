@@ -126,7 +126,10 @@ HostStage* take_stage(int device) {
     h->device = device;
     void *m = nullptr, *d = nullptr;
     const RelaxedCapture relaxed;
-    bool ok = hipHostMalloc(&m, 2 * kSlots * kSlotBytes + 256, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess;
+    // coherent by request, not by the runtime's default: the host reads rows and the error word after
+    // an event, and the kernels read rows written between launches, without a flush
+    bool ok = hipHostMalloc(&m, 2 * kSlots * kSlotBytes + 256,
+                            hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess;
     h->mem = static_cast<uint8_t*>(m);
     ok = ok && hipHostGetDevicePointer(&d, m, 0) == hipSuccess;
     h->dev = static_cast<uint8_t*>(d);

@@ -8,6 +8,7 @@
 //                               the failed calls' error is not taken for a launch's
 //   host_calls_test capture     sets are allocated and freed in the relaxed capture mode, also
 //                               the set of a call beyond those that stay idle
+#include <atomic>
 #include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
@@ -48,6 +49,7 @@ hipError_t alloc(void** p, size_t n) {
 }
 enum Fail { kNone, kHostMalloc, kHostPointer, kEvent };
 Fail g_fail = kNone;  // the call that fails
+std::atomic<bool> g_coherent{false};  // the last pinned allocation asked for coherent memory
 int g_copied_in = 0;  // rows or words copied to device memory
 }  // namespace
 
@@ -62,7 +64,8 @@ hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v 
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipMalloc(void** p, size_t n) { return alloc(p, n); }
 hipError_t hipFree(void* p) { return std::free(p), hipSuccess; }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+hipError_t hipHostMalloc(void** p, size_t n, unsigned flags) {
+    g_coherent = flags & hipHostMallocCoherent;
     if (g_fail == kHostMalloc) return err(hipErrorOutOfMemory);
     count(g_pinned, 1);
     return alloc(p, n);
@@ -157,7 +160,7 @@ int expect(bool ok, const char* what) {
 
 int at_exit() {
     if (expect(g_owner.open(4, 256, 256, 4) == QLIN_OK, "create")) return 1;
-    return expect(g_owner.run(4) == QLIN_OK, "run");
+    return expect(g_owner.run(4) == QLIN_OK, "run") | expect(g_coherent, "coherent memory");
 }
 
 int no_pinned() {
@@ -180,6 +183,7 @@ int no_pinned() {
 
 int capture() {
     constexpr int kCalls = 6, kIdle = 4;
+    std::atomic<int> failed{0};
     int bad = 0;
     {
         Pair p[kCalls];
@@ -187,11 +191,11 @@ int capture() {
             if (expect(x.open(4, 256, 256, 4) == QLIN_OK, "create")) return 1;
         g_gate = kCalls;  // every call holds a set of its own before any gives it back
         std::vector<std::thread> threads;
-        for (Pair& x : p) threads.emplace_back([&bad, &x] {
-            if (x.run(4) != QLIN_OK) bad = 1;
+        for (Pair& x : p) threads.emplace_back([&failed, &x] {
+            if (x.run(4) != QLIN_OK) failed = 1;
         });
         for (std::thread& t : threads) t.join();
-        bad |= expect(!bad, "runs") | expect(g_pinned == kIdle, "sets kept") | expect(!g_exposed, "sets given back");
+        bad |= expect(!failed, "runs") | expect(g_pinned == kIdle, "sets kept") | expect(!g_exposed, "sets given back");
     }
     return bad | expect(g_pinned == 0 && g_events == 0, "nothing kept without a workspace") |
            expect(!g_exposed, "sets freed with the last workspace");
