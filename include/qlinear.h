@@ -83,7 +83,8 @@ typedef struct qlin_workspace_info {
     int32_t max_rows;
     int32_t reserved;
     uint64_t device_bytes;      /* scratch: quantized rows, scales, split-K partials, counters */
-    uint64_t pinned_host_bytes; /* staging for the host-buffer entry points */
+    uint64_t pinned_host_bytes; /* staging of the host-buffer entry points now allocated; the process's
+                                   workspaces share it (0 before the first such call) */
 } qlin_workspace_info;
 
 /* Reference: rk_npu_strerror (src/npu.rs:138-144). */

@@ -75,6 +75,7 @@ namespace {
 // so calls on several threads and streams use different sets.
 constexpr int kSlots = 4;
 constexpr size_t kSlotBytes = (size_t)1 << 20;  // of rows in and of rows out
+constexpr size_t kSetBytes = 2 * kSlots * kSlotBytes + 256;
 constexpr int kIdleSets = 4;
 
 struct HostStage {
@@ -94,6 +95,7 @@ std::mutex& stage_mutex() {
 HostStage* g_idle[kIdleSets];  // idle sets, under stage_mutex as the counts
 int g_n_idle = 0;
 int g_workspaces = 0;          // live workspaces
+std::atomic<int> g_sets{0};    // sets allocated, idle or in a call
 
 // Keeps allocations and frees out of the checks of a graph that another thread records in global
 // capture mode.  (The copies and waits of a host-buffer call end such a capture all the same.)
@@ -107,7 +109,10 @@ void free_stage(HostStage* h) {
     const RelaxedCapture relaxed;
     for (hipEvent_t e : h->done)
         if (e) (void)hipEventDestroy(e);
-    if (h->mem) (void)hipHostFree(h->mem);
+    if (h->mem) {
+        (void)hipHostFree(h->mem);
+        --g_sets;
+    }
     delete h;
 }
 
@@ -128,9 +133,10 @@ HostStage* take_stage(int device) {
     const RelaxedCapture relaxed;
     // coherent by request, not by the runtime's default: the host reads rows and the error word after
     // an event, and the kernels read rows written between launches, without a flush
-    bool ok = hipHostMalloc(&m, 2 * kSlots * kSlotBytes + 256,
+    bool ok = hipHostMalloc(&m, kSetBytes,
                             hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess;
     h->mem = static_cast<uint8_t*>(m);
+    g_sets += m != nullptr;
     ok = ok && hipHostGetDevicePointer(&d, m, 0) == hipSuccess;
     h->dev = static_cast<uint8_t*>(d);
     for (int i = 0; ok && i < kSlots; ++i) ok = hipEventCreateWithFlags(&h->done[i], hipEventDisableTiming) == hipSuccess;
@@ -611,7 +617,7 @@ int qlin_workspace_query(const qlin_workspace* ws, qlin_workspace_info* out) {
     out->max_rows = ws->max_rows;
     out->reserved = 0;
     out->device_bytes = ws->device_bytes;
-    out->pinned_host_bytes = 0;
+    out->pinned_host_bytes = (uint64_t)g_sets.load() * kSetBytes;
     return QLIN_OK;
 }
 

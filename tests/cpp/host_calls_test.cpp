@@ -50,6 +50,7 @@ hipError_t alloc(void** p, size_t n) {
 enum Fail { kNone, kHostMalloc, kHostPointer, kEvent };
 Fail g_fail = kNone;  // the call that fails
 std::atomic<bool> g_coherent{false};  // the last pinned allocation asked for coherent memory
+std::atomic<size_t> g_pinned_bytes{0};  // of the last one
 int g_copied_in = 0;  // rows or words copied to device memory
 }  // namespace
 
@@ -66,6 +67,7 @@ hipError_t hipMalloc(void** p, size_t n) { return alloc(p, n); }
 hipError_t hipFree(void* p) { return std::free(p), hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned flags) {
     g_coherent = flags & hipHostMallocCoherent;
+    g_pinned_bytes = n;
     if (g_fail == kHostMalloc) return err(hipErrorOutOfMemory);
     count(g_pinned, 1);
     return alloc(p, n);
@@ -160,7 +162,12 @@ int expect(bool ok, const char* what) {
 
 int at_exit() {
     if (expect(g_owner.open(4, 256, 256, 4) == QLIN_OK, "create")) return 1;
-    return expect(g_owner.run(4) == QLIN_OK, "run") | expect(g_coherent, "coherent memory");
+    qlin_workspace_info info;
+    if (expect(qlin_workspace_query(g_owner.ws, &info) == QLIN_OK && info.pinned_host_bytes == 0, "no set yet")) return 1;
+    return expect(g_owner.run(4) == QLIN_OK, "run") | expect(g_pinned == 1, "one set") |
+           expect(qlin_workspace_query(g_owner.ws, &info) == QLIN_OK && info.pinned_host_bytes == g_pinned_bytes,
+                  "pinned bytes reported") |
+           expect(g_coherent, "coherent memory");
 }
 
 int no_pinned() {
