@@ -1148,6 +1148,21 @@ int run_host_copies(qlin_workspace* ws, const qlin_weights* w, int rows, const f
     return e ? QLIN_ERR_NONFINITE : QLIN_OK;
 }
 
+// Whether rows take longer in `blocks` pinned blocks than through device copies.  Every block
+// streams all the weights and goes through a product of its own, K long; the copies do that once,
+// but move the rows out at half the speed.  Two least-squares fits (7% and 13% rms) to 497 random
+// shapes timed both ways (K 64..32768, N 64..262144, 2..1024 rows, weights to 500 MB): us, W and
+// the rows in and out in MB.  With the 0.82, for the fits' error, one of those and of 366 shapes
+// that the fits had not seen takes 5% longer than through copies and none more; without the rule 41
+// of the 497 did, up to 2.1x.  W4 / W8 of 2560 x 151936 at 128 rows, a row a block: 5963 / 9549 us ->
+// 4586 / 4642; W8 28672 x 8192, 15 blocks: 1064 -> 758; W8 32160 x 190 at 212 rows, a long K: 1250 ->
+// 844; W4 2560 x 19456 at 128 rows, 10 blocks, stays at 358 (through copies 687).
+bool blocks_lag(const qlin_weights* w, int rows, int blocks, size_t row_in, size_t row_out) {
+    const double W = 1e-6 * w->N * w->wrow, in = 1e-6 * rows * row_in, out = 1e-6 * rows * row_out;
+    const double block_us = 0.9 + 0.43e-3 * w->K + 0.36 * std::max(0.4 * W, 19.0 * out / blocks);
+    return 21.0 + blocks * block_us + 25.5 * in + 30.0 * out > 0.82 * (58.0 + 0.256 * W + 32.6 * in + 55.0 * out);
+}
+
 // Host-buffer run in blocks of rows through pinned slots that the kernels read and write
 // themselves: the quantize launch reads a block's rows over the bus (each row once), the GEMM
 // stores its f32 rows straight into the slot, and while the GPU works on a block the host
@@ -1166,12 +1181,15 @@ int run_host(qlin_workspace* ws, const qlin_weights* w, int rows, const float* A
     const size_t row_in = (size_t)w->K * sizeof(float), row_out = (size_t)ncols * sizeof(float);
     const size_t per_slot = kSlotBytes / std::max(row_in, row_out);
     // rows whose quantization would read them by elements, or longer than a slot; buffers that
-    // overlap, where a block's rows out could land on rows that are still to go in; a thread on
-    // another device, whose events this stream could not record
+    // overlap, where a block's rows out could land on rows that are still to go in; weights that
+    // cost more to stream for every block than the blocks save; a thread on another device, whose
+    // events this stream could not record
     const uintptr_t a0 = reinterpret_cast<uintptr_t>(A), c0 = reinterpret_cast<uintptr_t>(C);
     const bool overlap = a0 < c0 + (size_t)rows * row_out && c0 < a0 + (size_t)rows * row_in;
+    const int blocks = per_slot ? (int)((rows + per_slot - 1) / per_slot) : 0;
     int device = -1;
-    if (w->K % 8 || per_slot == 0 || overlap || hipGetDevice(&device) != hipSuccess || device != ws->device)
+    if (w->K % 8 || blocks == 0 || overlap || blocks_lag(w, rows, blocks, row_in, row_out) ||
+        hipGetDevice(&device) != hipSuccess || device != ws->device)
         return run_host_copies(ws, w, rows, A, C, ncols, flags);
     HostStage* h = take_stage(ws->device);
     if (!h) return run_host_copies(ws, w, rows, A, C, ncols, flags);
@@ -1179,7 +1197,7 @@ int run_host(qlin_workspace* ws, const qlin_weights* w, int rows, const float* A
     ws->last = st;
     uint32_t* err_host = reinterpret_cast<uint32_t*>(h->mem + 2 * kSlots * kSlotBytes);
     *err_host = 0;
-    const int blocks = (int)((rows + per_slot - 1) / per_slot), step = (rows + blocks - 1) / blocks;
+    const int step = (rows + blocks - 1) / blocks;
     int rc = QLIN_OK;
     // the workspace's word reports this call, as every host-buffer call's
     if (ws->err_used && hipMemsetAsync(ws->err, 0, sizeof(uint32_t), st) != hipSuccess) rc = QLIN_ERR_DEVICE;

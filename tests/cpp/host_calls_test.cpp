@@ -8,6 +8,8 @@
 //                               the failed calls' error is not taken for a launch's
 //   host_calls_test capture     sets are allocated and freed in the relaxed capture mode, also
 //                               the set of a call beyond those that stay idle
+//   host_calls_test blocks      rows go through pinned blocks only where the weights, which every
+//                               block streams again, cost less than the blocks save
 #include <atomic>
 #include <condition_variable>
 #include <cstdio>
@@ -51,6 +53,7 @@ enum Fail { kNone, kHostMalloc, kHostPointer, kEvent };
 Fail g_fail = kNone;  // the call that fails
 std::atomic<bool> g_coherent{false};  // the last pinned allocation asked for coherent memory
 std::atomic<size_t> g_pinned_bytes{0};  // of the last one
+std::atomic<int> g_launches{0};
 int g_copied_in = 0;  // rows or words copied to device memory
 }  // namespace
 
@@ -123,7 +126,14 @@ hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
     *m = was;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t* st) {
+    *g = *b = dim3(1);
+    *lds = 0;
+    *st = nullptr;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) { return ++g_launches, hipSuccess; }
 }
 
 namespace {
@@ -208,11 +218,32 @@ int capture() {
            expect(!g_exposed, "sets freed with the last workspace");
 }
 
+int blocks() {
+    const struct {
+        int bits, K, N, rows, blocks;  // 0: one run through copies
+    } cases[] = {
+        {4, 2560, 6144, 128, 4},   {4, 4096, 2560, 128, 2},  {4, 2560, 19456, 128, 10}, {4, 9728, 2560, 128, 5},
+        {8, 2560, 19456, 8, 1},    {4, 2560, 151936, 1, 1},  {4, 2560, 151936, 32, 0},  {8, 8192, 28672, 64, 0},
+        {8, 32160, 192, 212, 0},
+    };
+    int bad = 0;
+    for (const auto& c : cases) {
+        Pair p;
+        if (expect(p.open(c.bits, c.K, c.N, c.rows) == QLIN_OK, "create")) return 1;
+        g_launches = g_copied_in = 0;
+        bad |= expect(p.run(c.rows) == QLIN_OK, "run");
+        const bool ok = c.blocks ? g_launches == 2 * c.blocks && g_copied_in == 0 : g_launches <= 2 && g_copied_in == 1;
+        if (!ok) std::printf("W%d %d x %d, %d rows: %d launches, %d copies in\n", c.bits, c.K, c.N, c.rows, (int)g_launches, g_copied_in);
+        bad |= expect(ok, "route");
+    }
+    return bad;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::string mode = argc > 1 ? argv[1] : "";
-    const int rc = mode == "exit" ? at_exit() : mode == "no_pinned" ? no_pinned() : mode == "capture" ? capture() : expect(false, "mode");
+    const int rc = mode == "exit" ? at_exit() : mode == "no_pinned" ? no_pinned() : mode == "capture" ? capture() : mode == "blocks" ? blocks() : expect(false, "mode");
     if (!rc) std::printf("PASS %s\n", mode.c_str());
     std::fflush(stdout);
     return rc;

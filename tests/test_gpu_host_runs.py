@@ -29,6 +29,7 @@ def weights(bits, K, N, seed):
     (4, 2560, 6144, 1), (4, 9728, 2560, 26), (4, 9728, 2560, 27), (8, 4096, 2560, 300), (4, 2560, 2000, 1000),
     (8, 64, 262144, 5),         # one row per block
     (8, 64, 262146, 3),         # a row longer than a slot
+    (8, 8192, 28672, 64), (8, 32160, 190, 212),  # weights, or a K, that cost more per block than it saves
     (8, 1001, 98, 40), (4, 1002, 98, 1)])
 def test_host_runs_equal_device_runs(bits, K, N, rows):
     w, ws = weights(bits, K, N, 960 + rows), ql.Workspace(rows, K, N)

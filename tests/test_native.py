@@ -28,7 +28,7 @@ def test_npu_mirror_host_logic():
     _run("cpu", 60)
 
 
-@pytest.mark.parametrize("mode", ["exit", "no_pinned", "capture"])
+@pytest.mark.parametrize("mode", ["exit", "no_pinned", "capture", "blocks"])
 def test_host_calls(mode):
     assert f"PASS {mode}" in _run_bin(HOST_BIN, mode, 60)
 
