@@ -646,7 +646,7 @@ int qlin_quantize(int32_t rows, int32_t K, const void* A, int32_t a_dtype, int64
     p.err = err;
     p.gamma = gamma;
     p.eps = eps;
-    p.flags = flags;
+    p.flags = flags & ~kFlagErrOnHost;
     return launch_quant(p, rows, (hipStream_t)stream) == hipSuccess ? QLIN_OK : QLIN_ERR_DEVICE;
 }
 
@@ -1124,7 +1124,7 @@ int run_impl(qlin_workspace* ws, const qlin_weights* w, int rows, const void* A,
     qp.err = ws->err;
     qp.gamma = gamma;
     qp.eps = eps;
-    qp.flags = flags;
+    qp.flags = flags & ~kFlagErrOnHost;
     if (launch_quant(qp, rows, st) != hipSuccess) return QLIN_ERR_DEVICE;
     return run_rows(ws, w, rows, ws->q, w->Kp, ws->s, C, c_dtype == QLIN_F16, ldc, flags, st, res);
 }
@@ -1222,8 +1222,7 @@ int run_host(qlin_workspace* ws, const qlin_weights* w, int rows, const float* A
         qp.q = ws->q;
         qp.s = ws->s;
         qp.err = reinterpret_cast<uint32_t*>(h->dev + 2 * kSlots * kSlotBytes);
-        qp.err_on_host = 1;
-        qp.flags = flags;
+        qp.flags = flags | kFlagErrOnHost;
         if (launch_quant(qp, m, st) != hipSuccess) rc = QLIN_ERR_DEVICE;
         if (!rc) rc = run_rows(ws, w, m, ws->q, w->Kp, ws->s, h->dev + out, 0, ncols, flags, st);
         if (!rc && hipEventRecord(h->done[slot], st) != hipSuccess) rc = QLIN_ERR_DEVICE;

@@ -47,7 +47,7 @@ __device__ __forceinline__ void quant8(const float v[8], float inv, bool rne, bo
 // is used, and an atomic on host memory would need the bus to carry it.
 __device__ __forceinline__ void flag_nonfinite(const QuantParams& p) {
     if (!p.err) return;
-    if (p.err_on_host) __hip_atomic_store(p.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (p.flags & kFlagErrOnHost) __hip_atomic_store(p.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     else atomicOr(p.err, 1u);
 }
 
@@ -557,28 +557,34 @@ __global__ __launch_bounds__(256) void quant_rows_reg_kernel(QuantParams p, int 
     }
     const float s = qscale_from_absmax(m);
     const float inv = 1.0f / s;
-    const bool rne = (p.flags & kFlagRne) != 0;
-    const bool fast = !bad;  // finite row: the short rounding sequence
     int8_t* qrow = p.q + (int64_t)row * p.ldq;
+    // The rounding is the row's: chosen once, not per group of four, where the compiler left every
+    // group a branch (12 x 11776 f32 rows 4.9 us, 4.4 so).
+    auto store = [&](auto rne, auto fast) {
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        const int c = lane + L * i;
-        if (c < nchunks) {
-            const T* e = reinterpret_cast<const T*>(&raw[i]);
-            uint32_t w[E / 4];
+        for (int i = 0; i < NC; ++i) {
+            const int c = lane + L * i;
+            if (c < nchunks) {
+                const T* e = reinterpret_cast<const T*>(&raw[i]);
+                uint32_t w[E / 4];
 #pragma unroll
-            for (int g = 0; g < E / 4; ++g) {
-                float v[4];
+                for (int g = 0; g < E / 4; ++g) {
+                    float v[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = lds_ld(e, 4 * g + j);
-                w[g] = quant4(v, inv, rne, fast);
+                    for (int j = 0; j < 4; ++j) v[j] = lds_ld(e, 4 * g + j);
+                    w[g] = quant4(v, inv, rne, fast);
+                }
+                if constexpr (E == 8)
+                    *reinterpret_cast<uint2*>(qrow + c * E) = make_uint2(w[0], w[1]);
+                else
+                    *reinterpret_cast<uint32_t*>(qrow + c * E) = w[0];
             }
-            if constexpr (E == 8)
-                *reinterpret_cast<uint2*>(qrow + c * E) = make_uint2(w[0], w[1]);
-            else
-                *reinterpret_cast<uint32_t*>(qrow + c * E) = w[0];
         }
-    }
+    };
+    const bool rne = (p.flags & kFlagRne) != 0;
+    if (bad) store(rne, std::false_type{});
+    else if (rne) store(std::true_type{}, std::true_type{});  // finite row: the short rounding sequence
+    else store(std::false_type{}, std::true_type{});
     for (int k0 = p.K + 8 * lane; k0 < p.ldq; k0 += 8 * L) *reinterpret_cast<uint2*>(qrow + k0) = make_uint2(0, 0);
     if (lane == 0) {
         p.s[row] = s;

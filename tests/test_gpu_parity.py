@@ -94,6 +94,26 @@ def test_quantize_nonfinite_flag(oracle):
     assert int(err.item()) == 0
 
 
+# plain rows of every instance (values per lane), rows with Inf / NaN among finite ones, which take
+# the long rounding sequence; the error word keeps its other bits, and a bit of flags that is
+# none of the entry point's changes nothing
+@pytest.mark.parametrize("dtype,K", [(torch.float32, K) for K in (512, 4096, 4104, 8192, 11776, 20480)] +
+                         [(torch.float16, K) for K in (1000, 8192, 9728, 16384, 40960)])
+@pytest.mark.parametrize("rne", [False, True])
+def test_quantize_plain_rows_nonfinite(oracle, dtype, K, rne):
+    x = synth.activations(6, K, seed=K + 9, device="cpu", dist="student_t3").to(dtype)
+    x[1, 3], x[3, K - 1], x[4] = float("nan"), float("-inf"), 0.0
+    flags = (ql.QLIN_ROUND_HALF_EVEN if rne else 0) | 0x80000000
+    err = torch.full((1,), 0x50, dtype=torch.int32, device=DEV)
+    q, s = ql.quantize(x.to(DEV), ldq=roundup(K, 256) + 256, flags=flags, err=err)
+    torch.cuda.synchronize()
+    qo, so, bad = oracle.quantize(x.float().numpy(), oracle.ROUND_EVEN if rne else oracle.ROUND_AWAY)
+    assert bad == 2 and int(err.item()) == 0x51
+    fine = np.isfinite(x.float().numpy()).all(1)
+    assert np.array_equal(s.cpu().numpy().view(np.uint32)[fine], so.view(np.uint32)[fine])
+    assert np.array_equal(q.cpu().numpy()[:, :K], qo) and not q.cpu().numpy()[:, K:].any()
+
+
 @pytest.mark.parametrize("order", ["neon16", "seq"])
 @pytest.mark.parametrize("M,K", [(1, 2560), (5, 100), (3, 9728), (33, 4096)])
 def test_rmsnorm_quantize_bitexact(oracle, order, M, K):
