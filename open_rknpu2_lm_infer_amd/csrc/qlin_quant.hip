@@ -362,6 +362,11 @@ static bool launch_quant_block(const QuantParams& p, int rows, hipStream_t strea
     if (chunks > 2048 || lds > (size_t)kStageBytes || (p.flags & kFlagNormSeq) || p.K % (64 * E))
         return false;
     const int nc = chunks > 1024 ? 2 : 1, threads = ((chunks + nc - 1) / nc + 63) / 64 * 64;
+    // one round of workgroups on the 256 CUs (2048 threads, 160 KiB of LDS each): in a second round the
+    // staged kernel's smaller workgroups are ahead (f32 701 / 939 rows of 4096: 8.0 / 8.8 us, here 8.8 /
+    // 10.1; over 256 random shapes of 200..1023 rows this takes 0.79 of its time in one round, 1.04 in two)
+    const int per_cu = std::min(2048 / threads, (int)(160 * 1024 / (lds + 128)));
+    if (rows > 256 * per_cu) return false;
     if (nc == 1) quant_norm_block_kernel<T, 1><<<dim3(rows), dim3(threads), lds, stream>>>(p);
     else quant_norm_block_kernel<T, 2><<<dim3(rows), dim3(threads), lds, stream>>>(p);
     return true;

@@ -208,11 +208,13 @@ def test_rmsnorm_quantize_many_rows_nonfinite(oracle, dtype, K):
 
 # RMSNorm rows below 1024, a workgroup per row: one and two 16-byte chunks per thread (K up to
 # 8192 fp16 / 4096 f32, then twice that), the smallest K of each type, a K whose chunks do not
-# fill the last wave, the longest rows, one row and the most rows of its range
+# fill the last wave, the longest rows, one row, and the most rows that one round of workgroups
+# takes (in the call with three rows more the staged kernel)
 @pytest.mark.parametrize("dtype,K,M", [
     (torch.float16, 512, 3), (torch.float16, 2560, 1023), (torch.float16, 8192, 2), (torch.float16, 8704, 5),
     (torch.float16, 16384, 1), (torch.float32, 256, 3), (torch.float32, 2560, 300), (torch.float32, 4096, 1),
-    (torch.float32, 4352, 5), (torch.float32, 8192, 2)])
+    (torch.float32, 4352, 5), (torch.float32, 8192, 2), (torch.float32, 4096, 512), (torch.float32, 5120, 768),
+    (torch.float16, 6656, 512)])
 def test_rmsnorm_quantize_row_per_workgroup(oracle, dtype, K, M):
     x = synth.activations(M + 3, K, seed=K + 5, device="cpu", dist="student_t3").to(dtype)
     x[M, 7], x[M + 1, K - 1], x[M + 2] = float("nan"), float("-inf"), 0.0
