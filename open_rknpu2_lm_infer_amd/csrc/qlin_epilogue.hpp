@@ -1,5 +1,5 @@
-// Dequant / SiLU-gate / residual epilogue of four consecutive output channels of one row,
-// shared by the GEMM kernels whose lanes hold their int32 sums that way.
+// Shared by the GEMM kernels whose lanes hold the int32 sums of four consecutive output channels of
+// one row: the order of the tiles and the dequant / SiLU-gate / residual epilogue.
 #pragma once
 
 #include "qlin_internal.hpp"
@@ -7,6 +7,18 @@
 namespace qlin {
 
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+
+// Tile of workgroup b of n, in contiguous ranges per XCD (workgroups go round the eight XCDs), so that
+// the tiles of a column find its weights in one L2; the first n % 8 ranges are one longer.  (With ranges
+// only where 8 divides n, 189 tiles of the wave-split-K GEMM, 200 rows of W4 4096 x 2560, took 12.0 us;
+// 9.7 so.  W8 9728 x 2560 at 100 rows, 189 tiles: 28.6 and 15.4.)  Columns of one tile have no weights
+// to share, and keep the plain order where 8 does not divide n: W8 2560 x 19456 with SiLU-gate at 32 rows,
+// 203 tiles, 14.0 us, in ranges 14.7.
+__device__ __forceinline__ int xcd_tile(int b, int n, int m_tiles) {
+    const int x = b & 7;
+    if (m_tiles == 1 && (n & 7)) return b;
+    return x * (n >> 3) + min(x, n & 7) + (b >> 3);
+}
 
 // Whether the rows of C / R take one vector access per four channels.
 __device__ __forceinline__ bool c_rows_vec(const GemmParams& p) {

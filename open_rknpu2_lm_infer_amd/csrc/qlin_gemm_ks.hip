@@ -96,9 +96,7 @@ __global__ __launch_bounds__(64 * WK) void gemm_ks_kernel(GemmParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 15, lc = lane >> 4;
 
-    const int NG = p.m_tiles * p.n_tiles;
-    int b = blockIdx.x;
-    if ((NG & 7) == 0) b = (b & 7) * (NG >> 3) + (b >> 3);  // contiguous tile ranges per XCD
+    const int b = xcd_tile(blockIdx.x, p.m_tiles * p.n_tiles, p.m_tiles);
     const int nt = b / p.m_tiles, mt = b - nt * p.m_tiles;
     const int m0 = mt * G::TM;
     constexpr int TC = SWIGLU ? G::TN / 2 : G::TN;  // output channels of the tile

@@ -116,10 +116,12 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_pp_kernel(GemmParams p) {
     constexpr int TC = SWIGLU ? BN / 2 : BN;  // output channels of a tile
     const int nh = p.N >> 1, ncols = SWIGLU ? nh : p.N;
 
-    // tiles of this workgroup: every `stride`-th of a contiguous range per XCD
+    // tiles of this workgroup: one, or every `stride`-th of a contiguous range per XCD
     const int NT = p.m_tiles * p.n_tiles, NG = gridDim.x;
     int tile = blockIdx.x, stride = NG, tile_end = NT;
-    if ((NG & 7) == 0) {
+    if (NT == NG) {
+        tile = xcd_tile(tile, NT, p.m_tiles);
+    } else if ((NG & 7) == 0) {
         const int per = (NT + 7) >> 3, x = tile & 7;
         stride = NG >> 3;
         tile_end = min(NT, (x + 1) * per);
