@@ -250,14 +250,14 @@ int qlin_swiglu(int32_t rows, int32_t F, const void* X, int32_t x_dtype, int64_t
  * No counterpart in the reference, whose library reports its strategy through
  * rk_npu_w4a8_query / backend stats (src/npu.rs:631-661). */
 #define QLIN_PATH_GEMV_FUSED 0 /* one GEMV launch that quantizes (and normalizes) its rows itself */
-#define QLIN_PATH_GEMV 1       /* a quantize launch, then the GEMV or (tile_m > 0) the wave-split-K
-                                  GEMM on the quantized rows */
-#define QLIN_PATH_GEMM 2       /* a quantize launch, then the tiled or the wave-split-K MFMA GEMM */
+#define QLIN_PATH_GEMV 1       /* a quantize launch, then the GEMV or (tile_m > 0) the wave-split-K or
+                                  the alternating-waves MFMA GEMM on the quantized rows */
+#define QLIN_PATH_GEMM 2       /* a quantize launch, then one of those GEMMs or the tiled one */
 typedef struct qlin_plan {
     int32_t path;       /* QLIN_PATH_* */
     int32_t launches;   /* kernel launches of the call */
     int32_t waves;      /* waves per workgroup of the GEMV / GEMM */
-    int32_t item_width; /* GEMV, wave-split-K GEMM: output channels per item / tile */
+    int32_t item_width; /* GEMV: output channels per item; wave-split-K, alternating-waves GEMM: per tile */
     int32_t items;      /* GEMV items, or GEMM output tiles */
     int32_t grid;       /* workgroups of the GEMV / GEMM launch */
     int32_t splits;     /* GEMM: k splits per tile */
@@ -273,7 +273,7 @@ int qlin_run_plan(const qlin_workspace* ws, const qlin_weights* weights, int32_t
  * src/cli/tune.rs:10-59).  qlin_tune times, on `stream`, the variants of the path a run of
  * `rows` rows takes (decode GEMV: 4, 8 or 16 waves per channel group; GEMM: the 16x16x64
  * kernel and each tile configuration of the 32x32x32 kernel, each with 1..8 k splits) and the
- * planner's own wave-split-K kernel where it would run, checks that they all produce the same
+ * planner's own wave-split-K or alternating-waves kernel where that would run, checks that they all produce the same
  * output, and records the fastest variant for the key (bits, K, N, rows bucket, path,
  * QLIN_SWIGLU); later runs with that key use it, or keep the planner's kernel if that was
  * faster still.  The table is

@@ -359,12 +359,13 @@ int upload_scales(qlin_weights* x, const float* scales, hipMemcpyKind kind, hipS
     return QLIN_OK;
 }
 
-// Whether the decode GEMV takes the rows (else quantize + GEMM).  17..32 rows go through
-// the GEMV's two row blocks where it measured faster than the GEMM: every shape up to 20
-// rows, and up to 32 for outputs of at most 4096 channels, whose GEMM grid is a few wide
-// tiles split along K (W4 layer, µs per linear with its quantize launch, GEMM -> GEMV: o /
-// down at 17 rows 14.3 / 18.9 -> 9.4 / 14.0, at 32 rows 14.4 / 19.1 -> 10.6 / 17.5; qkv /
-// gate_up at 17 rows 14.7 / 16.4 -> 14.1 / 14.5, at 32 rows 14.8 / 16.5 -> 16.6 / 17.8).
+// Whether the rows go to the GEMV, or else to the tiled GEMM, where plan_rows leaves them to one of the
+// two; it also names the path that qlin_run_plan reports and the variant table's key.  17..32 rows go
+// through the GEMV's two row blocks where it measured faster than the tiled GEMM: every shape up to 20
+// rows, and up to 32 for outputs of at most 4096 channels, whose GEMM grid is a few wide tiles split
+// along K (W4 layer, us per linear with its quantize launch, tiled GEMM -> GEMV: o / down at 17 rows 14.3 /
+// 18.9 -> 9.4 / 14.0, at 32 rows 14.4 / 19.1 -> 10.6 / 17.5; qkv / gate_up at 17 rows 14.7 / 16.4 -> 14.1 /
+// 14.5, at 32 rows 14.8 / 16.5 -> 16.6 / 17.8).
 bool gemv_ok(const qlin_workspace* ws, const qlin_weights* w, int rows) {
     (void)ws;
     if (rows <= kGemvMaxRows) return true;
@@ -773,14 +774,14 @@ struct GemmPlan {
     int kernel;  // 32: the 32x32x32 kernel (tile configuration cfg), 16: the 16x16x64 kernel
     int cfg, bm, bn, threads;
     int m_tiles, n_tiles, splits, ktiles_per_split, group_m, deep, wn;
-    double est;  // estimated us of the k loop and the split exchange (0: splits forced)
 };
 
 // Kernel and tile configuration for a shape.  Measured (MI355X, four Qwen3-4B linears, M = 512
 // and 4096, fp16 out): the 32x32x32 kernel's 256 x 256 tile is ahead only where it leaves
 // every CU several tiles (M = 4096 gate_up: 194-206 vs 212-227 us); with one round or less
 // the 16x16x64 kernel is equal or ahead (M = 512: the 128 x 128 tiles of both run at the
-// same copy rate, ~20 B per clock per CU), so it stays the default there.
+// same copy rate, ~20 B per clock per CU), so it stays the default there.  (Where this picks the 32x32x32
+// kernel without an override or a table entry, plan_rows takes the alternating-waves GEMM instead.)
 // Returns -1 for the 16x16x64 kernel, else the 32x32x32 tile configuration.  `tuned` is the
 // kernel field of a variant-table entry (0: none), below the environment overrides.
 int gemm_pick(const qlin_workspace* ws, const qlin_weights* w, int rows, bool sw, int tuned) {
@@ -861,7 +862,6 @@ int plan_gemm(const qlin_workspace* ws, const qlin_weights* w, int rows, uint32_
                 S = t;
             }
         }
-        g.est = best;
     }
     S = std::max(1, std::min(S, ktiles));
     while (S > 1 && ((int64_t)tiles * S * slice > ws->part_ints || tiles > ws->n_counters)) --S;
@@ -930,40 +930,98 @@ RowsPlan rows_tiles(RowsPlan::Kind kind, int cfg, int bm, int bn, int waves, con
     return r;
 }
 
-// Where the wave-split-K estimate is too low, over 6084 random shapes (K 384..9728, N 256..19456,
-// 9..4096 rows, both kernels timed): large tiles over a K of at most six steps, whose epilogue is
-// most of the launch (68 shapes, the others in 0.96 of its geometric mean; W4 K =
-// 512, N = 7680, 167 rows 7.7 -> 6.5 us); W8 tiles of 96 channels over 36 steps and more (15
-// shapes, 0.91; K = 8576, N = 2944, 219 rows 30.3 -> 18.3); and tiles of 64 and more rows over as
-// many steps above 1792 rows, where every workgroup of a row block streams the same long rows (0.91;
-// W8 K = 6400, N = 384, 2728 rows 26.5 -> 18.1).  By tile height and K it takes 0.4..1.0 elsewhere.
-bool gemm_ks_lags(const KsTile& t, int steps, int rows, bool w4) {
-    if (steps <= 6) return t.mf * t.nb >= (w4 ? 20 : 18);
-    return steps >= 36 && ((!w4 && t.nb == 6) || (t.mf >= 4 && rows > 1792));
+// Estimates of a launch on quantized rows, in us, behind the choice of its kernel.  Each is a sum of
+// what the kernel does, with the factors of W4 and W8: least squares of the relative error to half of
+// 12814 random shapes (K 64..32768, N 64..262144, 1..8192 rows, a third with SiLU-gate, fp16 out, up to
+// eight copies of the weights in turn), each timed in graphs with every kernel and configuration that
+// takes it.  rms error over the other half: wave-split-K 7.4%, alternating 5..7%, tiled 7..10%, GEMV
+// 11..18%.
+struct RowsCost {
+    int rows, steps;          // 128-deep k steps
+    double w, q, out, odd;    // MB: weights, quantized rows, fp16 outputs; outputs in rows not a multiple of 4
+    int b;                    // 0: W4, 1: W8
+    bool sw;
+};
+
+RowsCost rows_cost(const qlin_weights* w, int rows, bool sw) {
+    const int ncols = sw ? w->N / 2 : w->N;
+    RowsCost k{rows, w->Kp / 128, 1e-6 * w->N * w->wrow, 1e-6 * rows * w->Kp, 2e-6 * rows * ncols, 0.0, w->bits == 8, sw};
+    if (ncols % 4) k.odd = k.out;
+    return k;
 }
 
-// Which kernel takes quantized rows.
+// One round of workgroups: the KiB a workgroup copies (its rows and its weights), the partial sums'
+// exchange, the MFMAs, the operands of all workgroups, the outputs, the weights and the rows once.
+// Over more than 96 steps it comes out low (by a tenth at 128..255).
+double ks_us(const RowsCost& k, const KsTile& t, int m_tiles, int n_tiles) {
+    static constexpr double c[2][9] = {{3.54, 0.00329, 0.0112, 0.0142, 0.00306, 0.00825, 1.13, 0.0760, 0.139},
+                                       {3.52, 0.00408, 0.00708, 0.0184, 0.00193, 0.00964, 0.830, 0.103, 0.190}};
+    const double* f = c[k.b];
+    const double own = (k.steps + t.wk - 1) / t.wk;  // k steps of the busiest wave
+    const double us = f[0] + t.wk * own * (f[1] * 2 * t.mf + f[2] * t.nb * (1 + k.b)) +
+                      t.wk * t.mf * t.nb * (f[3] + f[4] * own) + f[5] * (n_tiles * k.q + m_tiles * k.w) + f[6] * k.out +
+                      f[7] * k.w + f[8] * k.q;
+    return (k.steps > 96 ? 1.12 : 1.0) * t.rel[k.b] * us;
+}
+
+// Rounds of tiles at the configuration's cost per tile and k step, the weights once, the outputs (more
+// where their rows take narrow stores), the operands of all tiles.  1.015: it comes out 1% low.
+double pp_us(const RowsCost& k, const PpTile& t, int tiles, int cus) {
+    static constexpr double c[2][5] = {{3.30, 0.0157, 0.156, 0.580, 0.0118}, {3.06, 0.0628, 0.164, 0.598, 0.00963}};
+    const double* f = c[k.b];
+    const int rounds = tiles / cus + (tiles % cus != 0);
+    const double operands = 128e-6 * tiles * k.steps * (t.bm + 0.5 * t.bn * (1 + k.b));
+    return 1.015 * (f[0] + rounds * (t.tile_us[k.b] + k.steps * t.step_us[k.b]) + f[1] * k.w + f[2] * k.out +
+                    f[3] * k.odd + f[4] * operands);
+}
+
+// The 16x16x64 tiled GEMM, unsplit or with K split over workgroups: rounds of k steps, workgroups per
+// CU, operands, outputs, then the splits' exchange through memory, the weights and the rows once.
+double tiled_us(const RowsCost& k, const GemmPlan& g, int cus) {
+    static constexpr double c[2][2][10] = {{{4.78, 0.360, 0.216, 0.00797, 0.346, 0.542, 0.0, 0.0, 0.0312, 0.0583},
+                                            {5.87, 0.349, 0.0, 0.00480, 0.738, 1.69, 0.665, 0.143, 0.0266, 0.0424}},
+                                           {{4.24, 0.422, 1.38, 0.0132, 0.364, 0.554, 0.0, 0.0, 0.0313, 0.0},
+                                            {5.02, 0.458, 0.0, 0.0, 1.06, 1.81, 0.710, 0.101, 0.0586, 0.0325}}};
+    const double* f = c[k.b][g.splits > 1];
+    const double tiles = (double)g.m_tiles * g.n_tiles, wgs = tiles * g.splits;
+    const double operands = 128e-6 * tiles * k.steps * (g.bm + 0.5 * g.bn * (1 + k.b));
+    return f[0] + f[1] * std::ceil(wgs / cus) * g.ktiles_per_split + f[2] * wgs / cus + f[3] * operands + f[4] * k.out +
+           f[5] * k.odd + f[6] * g.splits + f[7] * 4e-6 * wgs * g.bm * g.bn + f[8] * k.w + f[9] * k.q;
+}
+
+// The GEMV on up to 8, 16 and 32 rows: rounds of the longest wave's steps (16 waves a CU), the weights,
+// the steps, the rows read for every 16 channels, the outputs, those channel groups, the second stream
+// of a SiLU-gate.  Over 4..7 of its own steps (256 deep for W4) it comes out 7% high.
+double gemv_us(const RowsCost& k, int N, int waves, int cus) {
+    static constexpr double c[2][3][8] = {{{3.28, 0.115, 0.143, 0.0229, 7.20, 5.60, 0.0331, 0.0157},
+                                           {3.34, 0.151, 0.0372, 0.0357, 22.2, 5.92, 0.0, 0.0078},
+                                           {4.05, 0.340, 0.185, 0.0427, 0.0, 3.97, 0.0, 0.0}},
+                                          {{2.86, 0.356, 0.118, 0.0265, 0.95, 4.55, 0.0, 0.0281},
+                                           {2.84, 0.425, 0.0691, 0.0379, 18.7, 3.88, 0.0, 0.0191},
+                                           {3.55, 0.520, 0.105, 0.0360, 0.342, 3.51, 0.0, 0.0264}}};
+    const double* f = c[k.b][k.rows <= 8 ? 0 : k.rows <= 16 ? 1 : 2];
+    const int groups = (N + 15) / 16, own = (k.steps + waves - 1) / waves;
+    const int64_t rounds = ((int64_t)groups * waves + 16 * cus - 1) / (16 * cus);
+    const double us = f[0] + f[1] * rounds * own + f[2] * k.w + f[3] * k.steps + f[4] * k.q * groups / cus +
+                      f[5] * k.out + f[6] * groups / cus + (k.sw ? f[7] * k.steps : 0.0);
+    const int deep = k.b ? k.steps : k.steps / 2;
+    return deep >= 4 && deep < 8 ? 0.93 * us : us;
+}
+
+// Which kernel takes quantized rows: the one with the least estimate among
+// - the wave-split-K GEMM in the configurations whose workgroups cover the output in one round, one per
+//   CU (most rings leave room for one; a second round costs a whole launch again: gate_up at 128 rows
+//   23.0 us in two rounds against 15.9 tiled),
+// - the alternating-waves GEMM, above 16 rows,
+// - what else takes the rows: the GEMV (gemv_ok) or the tiled GEMM.  Not its 32x32x32 kernel, whose
+//   tiles are the alternating kernel's and slower on every grid.
 //
-// Wave-split-K: a configuration is taken only where one round of workgroups covers the output
-// (its 160 KiB rings leave one workgroup per CU, and a second round costs a whole launch
-// again: gate_up at 128 rows 23.0 us in two rounds against 15.9 tiled).  Among those, the
-// least estimated time: a least-squares fit over 180 one-round measurements (five tile heights
-// x W4 / W8 x the four Qwen3-4B linears at 17..512 rows; 11% rms, and its pick within 1% of
-// the best measured on average) of a constant, the KiB a CU copies, the weight stream, the
-// partial sums' exchange and the MFMA steps.  Up to 32 rows, where the alternative is the GEMV
-// or a one-tile-high GEMM, that always won (qkv / o / gate_up / down at 16 rows 7.4 / 5.0 /
-// 10.9 / 8.6 us -> 4.2 / 4.1 / 9.3 / 7.7; at 8 rows 6.1 / 4.2 / 9.1 / 7.2 -> 4.1 / 4.0 / 9.0 /
-// 6.5).
-//
-// Above 32 rows it is compared with the alternating-waves GEMM (rounds of tiles at the
-// measured us per k step and per tile of each configuration) and with the tiled GEMM's own
-// estimate plus that kernel's fixed cost, whose split K keeps few tiles of a long K ahead:
-// down at 300 / 512 rows 19.8 / 21.7 us, unsplit 31.7 / 33.1.  o keeps the wave-split-K kernel
-// up to 512 rows (11.0 us; 16.0 alternating), qkv up to 256 (10.8; 12.1); qkv at 300 / 512 /
-// 1024 / 4096 rows tiled -> alternating 14.2 / 14.8 / 23.2 / 72.5 -> 12.0 / 12.6 / 19.6 / 58.1.
-// The 0.9 leaves split cases within the estimates' error (o at 640 rows: 15.8 tiled, 16.2
-// alternating) where they were.  W4 gate_up at 300 / 512 / 1024 / 4096 rows: 29.3 / 33.0 / 58.0 /
-// 195 -> 23.4 / 29.0 / 54.0 / 164; W8 qkv at 4096 112.7 -> 72.0, gate_up 300 -> 218.
+// Over 10269 further shapes the choice takes 1.011 times the best of all measured (geometric mean) and
+// 0.80 times the GEMV or the tiled GEMM alone; 2.0% of them are over 4% slower than those, 0.4% over
+// 10%, the worst 1.37x (K above 10000 into a few hundred channels).  W4 2560 x 6144 / 4096 x 2560 / 2560 x
+// 19456 / 9728 x 2560, GEMV or tiled -> chosen: 16 rows 8.2 / 5.7 / 11.3 / 9.0 us -> 5.0 / 5.0 / 8.5 / 6.5;
+// 128 rows 13.7 / 13.0 / 14.7 / 17.4 -> 8.6 / 7.3 / 14.1 / 11.3; 512 rows 16.0 / 15.3 / 32.6 / 22.3 -> 14.5 /
+// 12.3 / 30.2 / 20.7; 4096 rows 68.2 / 51.6 / 202 / 109 -> 59.9 / 43.5 / 164 / 84.
 //
 // Overrides of the GEMV's or the tiled GEMM's launch shape, and table entries, select those.
 RowsPlan plan_rows(const qlin_workspace* ws, const qlin_weights* w, int rows, int64_t ldq, uint32_t flags) {
@@ -990,57 +1048,33 @@ RowsPlan plan_rows(const qlin_workspace* ws, const qlin_weights* w, int rows, in
         ov.gemv_item_width > 0)
         return other;
     if (tuned_variant(w->bits, w->K, w->N, rows, gemv_ok(ws, w, rows) ? 1 : 2, sw)) return other;
-    const int steps = w->Kp / 128;
+    const RowsCost k = rows_cost(w, rows, sw);
+    const int cus = ws->cu_count;
     RowsPlan best = other;
     double best_us = 1e30;
+    if (gemv_ok(ws, w, rows)) {
+        best_us = gemv_us(k, w->N, plan_gemv(ws, w, rows, false, false, flags).waves, cus);
+    } else {
+        GemmPlan g;
+        if (plan_gemm(ws, w, rows, flags, &g)) return other;
+        if (g.kernel == 16) best_us = tiled_us(k, g, cus);
+    }
+    auto consider = [&](const RowsPlan& r, double us) {
+        if (us < best_us) {
+            best_us = us;
+            best = r;
+        }
+    };
     for (int c = 0; c < kKsConfigs && ov.gemm_ks != -2; ++c) {
         if (!ks_ok(c)) continue;
         const RowsPlan r = ks_plan(c);
-        if ((int64_t)r.m_tiles * r.n_tiles > ws->cu_count) continue;
-        const KsTile t = gemm_ks_tile(c);
-        const double own = (steps + t.wk - 1) / t.wk;  // k steps of the busiest wave
-        const double us = 1.7 + 0.0059 * t.wk * own * (2 * t.mf + t.nb * (w4 ? 1 : 2)) +
-                          0.25e-6 * ((double)w->N * w->wrow) + 0.0087 * t.wk * t.mf * t.nb +
-                          0.0066 * own * t.wk * t.mf * t.nb;
-        if (us < best_us) {
-            best_us = us;
-            best = r;
-        }
+        if ((int64_t)r.m_tiles * r.n_tiles <= cus) consider(r, ks_us(k, gemm_ks_tile(c), r.m_tiles, r.n_tiles));
     }
-    if (rows <= kGemvMaxRowsWide) return best;
-    if (best.kind == RowsPlan::kWaveSplitK && gemm_ks_lags(gemm_ks_tile(best.cfg), steps, rows, w4)) {
-        best = other;
-        best_us = 1e30;
-    }
-    GemmPlan g;
-    if (plan_gemm(ws, w, rows, flags, &g)) return other;
-    const int cus = ws->cu_count, rounds = (g.m_tiles * g.n_tiles + cus - 1) / cus;
-    // W4: two workgroups of the tiled GEMM share a CU, W8: one; the estimate's k step is W4's.
-    // Splitting more tiles than half the CUs gained nothing (o at 1024 rows, 160 tiles: 23.3 us
-    // with 1 or 2 splits).
-    const bool split = g.splits > 1 && 2 * g.m_tiles * g.n_tiles <= cus;
-    double tiled_us = split ? (w4 ? 1.0 : 1.15) * g.est + 4.5
-                            : (w4 ? 0.45 : 0.60) * steps + 6.0;
-    if (rounds > 1) tiled_us *= w4 ? 0.8 * rounds : rounds;
-    if (g.kernel == 32) tiled_us = 1e30;  // its tiles are the alternating kernel's, slower on every grid
-    if (best_us >= tiled_us) {
-        best = other;
-        best_us = (split ? 0.9 : 1.0) * tiled_us;
-    }
-    for (int c = 0; c < kPpConfigs && ov.gemm_pp != -2; ++c) {
+    for (int c = 0; c < kPpConfigs && ov.gemm_pp != -2 && rows > 16; ++c) {
         if (!pp_ok(c)) continue;
         const RowsPlan r = pp_plan(c);
-        const PpTile t = gemm_pp_tile(c);
-        const int n = (int)std::min<int64_t>(((int64_t)r.m_tiles * r.n_tiles + cus - 1) / cus, 1 << 20);
-        // a tile's fixed part grows with the share of CUs that store at once, and shrinks for
-        // the later rounds, whose first copies run under the previous tile's epilogue
-        const double load = 1.0 + 0.4 * r.m_tiles * r.n_tiles / ((double)n * cus);
-        const double us = n * steps * (w4 ? t.step_us : t.step8_us) + (0.25 + 0.75 * n) * t.tile_us * load +
-                          0.12e-6 * ((double)w->N * w->wrow);
-        if (us < best_us) {
-            best_us = us;
-            best = r;
-        }
+        const int64_t tiles = (int64_t)r.m_tiles * r.n_tiles;
+        if (tiles <= INT32_MAX) consider(r, pp_us(k, gemm_pp_tile(c), (int)tiles, cus));
     }
     return best;
 }

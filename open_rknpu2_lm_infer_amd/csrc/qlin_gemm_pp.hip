@@ -358,16 +358,19 @@ static hipError_t launch_c(const GemmParams& p, int cus, hipStream_t st) {
 }  // namespace pp
 
 // Tile configurations: tokens x weight rows, what each is built for, and the us per 128-deep k
-// step (W4, W8) and per tile behind the planner's estimate, measured with one round of
-// workgroups at K = 2560, 4096 and 9728.  Configuration 0 needs all 256 registers, and without
-// SiLU-gate it would spill; 6 is 5 with the waves laid out for SiLU-gate (each wave then needs
-// an even number of 16-row blocks).
+// step and per tile (W4, W8) of the planner's estimate, from its fit.  Configuration 0 needs all
+// 256 registers, and without SiLU-gate it would spill; 6 is 5 with the waves laid out for SiLU-gate
+// (each wave then needs an even number of 16-row blocks).
 constexpr PpTile kPpTiles[kPpConfigs] = {
-    // bm, bn, W4, W8, plain, SiLU-gate, us per k step W4, W8, us per tile
-    {256, 256, true, false, false, true, 1.07, 0.0, 8.4},  {256, 192, true, false, true, true, 0.87, 0.0, 8.3},
-    {256, 128, true, true, true, true, 0.58, 0.68, 6.4},   {128, 96, true, true, true, false, 0.38, 0.39, 4.1},
-    {128, 128, true, true, true, true, 0.41, 0.48, 4.0},   {128, 192, true, true, true, false, 0.55, 0.66, 4.5},
-    {128, 192, true, true, false, true, 0.60, 0.68, 5.0},  {128, 256, true, true, true, true, 0.63, 0.83, 6.0},
+    // bm, bn, W4, W8, plain, SiLU-gate, us per k step W4, W8, us per tile W4, W8
+    {256, 256, true, false, false, true, {1.03, 0}, {5.91, 0}},
+    {256, 192, true, false, true, true, {0.867, 0}, {4.61, 0}},
+    {256, 128, true, true, true, true, {0.562, 0.559}, {3.3, 3.09}},
+    {128, 96, true, true, true, false, {0.329, 0.332}, {1.92, 2.01}},
+    {128, 128, true, true, true, true, {0.355, 0.37}, {1.81, 1.74}},
+    {128, 192, true, true, true, false, {0.45, 0.505}, {3.16, 2.62}},
+    {128, 192, true, true, false, true, {0.512, 0.52}, {3.18, 2.47}},
+    {128, 256, true, true, true, true, {0.582, 0.607}, {3.53, 3.16}},
 };
 
 PpTile gemm_pp_tile(int cfg) { return kPpTiles[cfg]; }

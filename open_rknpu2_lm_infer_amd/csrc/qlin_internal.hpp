@@ -143,19 +143,21 @@ struct GemmTileCfg {
 };
 GemmTileCfg gemm32_tile(int bits, int cfg);
 hipError_t launch_gemm32(const GemmParams& p, int bits, int cfg, hipStream_t stream);
-// Tile configuration of the wave-split-K GEMM: row fragments and channel blocks of 16, waves along k.
+// Tile configuration of the wave-split-K GEMM: row fragments and channel blocks of 16, waves along k; its
+// time against the fit over all configurations (W4, W8).
 struct KsTile {
     int mf, nb, wk;
+    double rel[2];
 };
 constexpr int kKsConfigs = 20;
 KsTile gemm_ks_tile(int cfg);
 bool gemm_ks_fits(int bits, int cfg);  // two stages of every wave's ring fit the LDS
 hipError_t launch_gemm_ks(const GemmParams& p, int bits, int cfg, hipStream_t stream);
-// Tile of the alternating-waves GEMM: tokens x weight rows, what it is built for, its measured cost.
+// Tile of the alternating-waves GEMM: tokens x weight rows, what it is built for, its fitted cost.
 struct PpTile {
     int bm, bn;
     bool w4, w8, plain, swiglu;
-    double step_us, step8_us, tile_us;
+    double step_us[2], tile_us[2];  // W4, W8
 };
 constexpr int kPpConfigs = 8;
 PpTile gemm_pp_tile(int cfg);
