@@ -932,10 +932,10 @@ RowsPlan rows_tiles(RowsPlan::Kind kind, int cfg, int bm, int bn, int waves, con
 
 // Estimates of a launch on quantized rows, in us, behind the choice of its kernel.  Each is a sum of
 // what the kernel does, with the factors of W4 and W8: least squares of the relative error to half of
-// 12814 random shapes (K 64..32768, N 64..262144, 1..8192 rows, a third with SiLU-gate, fp16 out, up to
-// eight copies of the weights in turn), each timed in graphs with every kernel and configuration that
-// takes it.  rms error over the other half: wave-split-K 7.4%, alternating 5..7%, tiled 7..10%, GEMV
-// 11..18%.
+// 21152 random shapes (K 64..32768, N 64..262144, 1..8192 rows, a third with SiLU-gate, fp16 out), each
+// timed in graphs with every kernel and configuration that takes it, two thirds of them with eight copies
+// of the weights in turn, the others with copies beyond the 256 MB cache, as the layers of a model have
+// theirs.  rms error over the other half: wave-split-K 9%, alternating 5..7%, tiled 7..9%, GEMV 12..16%.
 struct RowsCost {
     int rows, steps;          // 128-deep k steps
     double w, q, out, odd;    // MB: weights, quantized rows, fp16 outputs; outputs in rows not a multiple of 4
@@ -954,8 +954,8 @@ RowsCost rows_cost(const qlin_weights* w, int rows, bool sw) {
 // exchange, the MFMAs, the operands of all workgroups, the outputs, the weights and the rows once.
 // Over more than 96 steps it comes out low (by a tenth at 128..255).
 double ks_us(const RowsCost& k, const KsTile& t, int m_tiles, int n_tiles) {
-    static constexpr double c[2][9] = {{3.54, 0.00329, 0.0112, 0.0142, 0.00306, 0.00825, 1.13, 0.0760, 0.139},
-                                       {3.52, 0.00408, 0.00708, 0.0184, 0.00193, 0.00964, 0.830, 0.103, 0.190}};
+    static constexpr double c[2][9] = {{3.08, 0.00383, 0.0127, 0.0154, 0.00245, 0.0115, 1.24, 0.0970, 0.119},
+                                       {3.14, 0.00479, 0.0080, 0.0195, 0.00154, 0.0147, 0.928, 0.105, 0.103}};
     const double* f = c[k.b];
     const double own = (k.steps + t.wk - 1) / t.wk;  // k steps of the busiest wave
     const double us = f[0] + t.wk * own * (f[1] * 2 * t.mf + f[2] * t.nb * (1 + k.b)) +
@@ -965,23 +965,23 @@ double ks_us(const RowsCost& k, const KsTile& t, int m_tiles, int n_tiles) {
 }
 
 // Rounds of tiles at the configuration's cost per tile and k step, the weights once, the outputs (more
-// where their rows take narrow stores), the operands of all tiles.  1.015: it comes out 1% low.
+// where their rows take narrow stores), the operands of all tiles.  1.008: it comes out that much low.
 double pp_us(const RowsCost& k, const PpTile& t, int tiles, int cus) {
-    static constexpr double c[2][5] = {{3.30, 0.0157, 0.156, 0.580, 0.0118}, {3.06, 0.0628, 0.164, 0.598, 0.00963}};
+    static constexpr double c[2][5] = {{3.16, 0.0182, 0.157, 0.581, 0.0133}, {2.97, 0.0654, 0.170, 0.598, 0.00819}};
     const double* f = c[k.b];
     const int rounds = tiles / cus + (tiles % cus != 0);
     const double operands = 128e-6 * tiles * k.steps * (t.bm + 0.5 * t.bn * (1 + k.b));
-    return 1.015 * (f[0] + rounds * (t.tile_us[k.b] + k.steps * t.step_us[k.b]) + f[1] * k.w + f[2] * k.out +
+    return 1.008 * (f[0] + rounds * (t.tile_us[k.b] + k.steps * t.step_us[k.b]) + f[1] * k.w + f[2] * k.out +
                     f[3] * k.odd + f[4] * operands);
 }
 
 // The 16x16x64 tiled GEMM, unsplit or with K split over workgroups: rounds of k steps, workgroups per
 // CU, operands, outputs, then the splits' exchange through memory, the weights and the rows once.
 double tiled_us(const RowsCost& k, const GemmPlan& g, int cus) {
-    static constexpr double c[2][2][10] = {{{4.78, 0.360, 0.216, 0.00797, 0.346, 0.542, 0.0, 0.0, 0.0312, 0.0583},
-                                            {5.87, 0.349, 0.0, 0.00480, 0.738, 1.69, 0.665, 0.143, 0.0266, 0.0424}},
-                                           {{4.24, 0.422, 1.38, 0.0132, 0.364, 0.554, 0.0, 0.0, 0.0313, 0.0},
-                                            {5.02, 0.458, 0.0, 0.0, 1.06, 1.81, 0.710, 0.101, 0.0586, 0.0325}}};
+    static constexpr double c[2][2][10] = {{{4.48, 0.354, 0.238, 0.0099, 0.345, 0.547, 0.0, 0.0, 0.0355, 0.0306},
+                                            {5.66, 0.355, 0.0, 0.00396, 0.744, 1.68, 0.658, 0.140, 0.0323, 0.0469}},
+                                           {{3.96, 0.450, 1.45, 0.00963, 0.365, 0.540, 0.0, 0.0, 0.0382, 0.0},
+                                            {4.89, 0.452, 0.0, 0.0, 1.15, 1.87, 0.704, 0.0967, 0.0661, 0.0320}}};
     const double* f = c[k.b][g.splits > 1];
     const double tiles = (double)g.m_tiles * g.n_tiles, wgs = tiles * g.splits;
     const double operands = 128e-6 * tiles * k.steps * (g.bm + 0.5 * g.bn * (1 + k.b));
@@ -993,12 +993,12 @@ double tiled_us(const RowsCost& k, const GemmPlan& g, int cus) {
 // the steps, the rows read for every 16 channels, the outputs, those channel groups, the second stream
 // of a SiLU-gate.  Over 4..7 of its own steps (256 deep for W4) it comes out 7% high.
 double gemv_us(const RowsCost& k, int N, int waves, int cus) {
-    static constexpr double c[2][3][8] = {{{3.28, 0.115, 0.143, 0.0229, 7.20, 5.60, 0.0331, 0.0157},
-                                           {3.34, 0.151, 0.0372, 0.0357, 22.2, 5.92, 0.0, 0.0078},
-                                           {4.05, 0.340, 0.185, 0.0427, 0.0, 3.97, 0.0, 0.0}},
-                                          {{2.86, 0.356, 0.118, 0.0265, 0.95, 4.55, 0.0, 0.0281},
-                                           {2.84, 0.425, 0.0691, 0.0379, 18.7, 3.88, 0.0, 0.0191},
-                                           {3.55, 0.520, 0.105, 0.0360, 0.342, 3.51, 0.0, 0.0264}}};
+    static constexpr double c[2][3][8] = {{{2.83, 0.111, 0.150, 0.0243, 7.47, 6.03, 0.0435, 0.0164},
+                                           {2.97, 0.0843, 0.122, 0.0397, 12.8, 5.99, 0.0, 0.00792},
+                                           {3.74, 0.301, 0.200, 0.0458, 0.0, 4.18, 0.0, 0.00271}},
+                                          {{2.48, 0.270, 0.130, 0.0341, 0.0, 4.78, 0.0120, 0.0291},
+                                           {2.49, 0.389, 0.0697, 0.0416, 22.7, 4.01, 0.0, 0.0203},
+                                           {3.09, 0.582, 0.125, 0.0303, 0.0, 3.61, 0.0, 0.0228}}};
     const double* f = c[k.b][k.rows <= 8 ? 0 : k.rows <= 16 ? 1 : 2];
     const int groups = (N + 15) / 16, own = (k.steps + waves - 1) / waves;
     const int64_t rounds = ((int64_t)groups * waves + 16 * cus - 1) / (16 * cus);
@@ -1016,12 +1016,12 @@ double gemv_us(const RowsCost& k, int N, int waves, int cus) {
 // - what else takes the rows: the GEMV (gemv_ok) or the tiled GEMM.  Not its 32x32x32 kernel, whose
 //   tiles are the alternating kernel's and slower on every grid.
 //
-// Over 10269 further shapes the choice takes 1.011 times the best of all measured (geometric mean) and
-// 0.80 times the GEMV or the tiled GEMM alone; 2.0% of them are over 4% slower than those, 0.4% over
-// 10%, the worst 1.37x (K above 10000 into a few hundred channels).  W4 2560 x 6144 / 4096 x 2560 / 2560 x
-// 19456 / 9728 x 2560, GEMV or tiled -> chosen: 16 rows 8.2 / 5.7 / 11.3 / 9.0 us -> 5.0 / 5.0 / 8.5 / 6.5;
-// 128 rows 13.7 / 13.0 / 14.7 / 17.4 -> 8.6 / 7.3 / 14.1 / 11.3; 512 rows 16.0 / 15.3 / 32.6 / 22.3 -> 14.5 /
-// 12.3 / 30.2 / 20.7; 4096 rows 68.2 / 51.6 / 202 / 109 -> 59.9 / 43.5 / 164 / 84.
+// Over 3449 further shapes the choice takes 1.013 times the best of all measured (geometric mean) and 0.80
+// times the GEMV or the tiled GEMM alone; 2.0% of them are over 4% slower than those, 0.4% over 10%, the
+// worst 1.23x. W4 2560 x 6144 / 4096 x 2560 / 2560 x 19456 / 9728 x 2560, GEMV or tiled -> chosen, us: 16
+// rows 8.0 / 5.7 / 11.2 / 9.0 -> 5.0 / 5.0 / 8.6 / 6.5; 128 rows 13.7 / 13.0 / 14.8 / 17.4 -> 8.7 / 7.3 /
+// 14.1 / 11.3; 512 rows 16.1 / 15.3 / 31.6 / 22.3 -> 14.6 / 12.4 / 28.8 / 22.3; 4096 rows 71.1 / 51.3 /
+// 198.6 / 107.4 -> 62.8 / 42.9 / 163.0 / 84.7.
 //
 // Overrides of the GEMV's or the tiled GEMM's launch shape, and table entries, select those.
 RowsPlan plan_rows(const qlin_workspace* ws, const qlin_weights* w, int rows, int64_t ldq, uint32_t flags) {

@@ -25,13 +25,13 @@
 // wave measured the same.  Per launch in a graph, quantized rows, eight copies of the weights in
 // turn, W4 (us, before -> chosen; before is the GEMV up to 20 rows and for o / down up to 32, else
 // the 128 x 128 GEMM; * another kernel than this one):
-//     rows      qkv 2560x6144    o 4096x2560     gate_up 2560x19456   down 9728x2560
-//     16         8.2 ->  5.0      5.7 ->  5.0    11.3 ->  8.5          9.0 ->  6.5
-//     24        12.1 ->  5.5      7.4 ->  5.3    13.0 ->  9.0         12.3 ->  7.4
-//     64        12.7 ->  6.6     12.1 ->  6.1    13.7 -> 11.5         16.3 ->  9.1
-//     128       13.7 ->  8.6     13.0 ->  7.3    14.7 -> 14.1*        17.4 -> 11.3
-//     300       15.0 -> 13.4*    14.7 -> 10.6    31.0 -> 21.9*        19.7 -> 17.3
-//     512       16.0 -> 14.5*    15.3 -> 12.3    32.6 -> 30.2*        22.3 -> 20.7
+//     rows qkv 2560x6144      o 4096x2560        gate_up 2560x19456 down 9728x2560
+//     16   8.0 ->  5.0        5.7 ->  5.0        11.2 ->  8.6       9.0 ->  6.5
+//     24   12.0 ->  5.5       7.4 ->  5.3        12.9 ->  9.1       12.2 ->  7.4
+//     64   12.7 ->  6.6       12.1 ->  6.2       13.8 -> 11.4       16.3 ->  9.1
+//     128  13.7 ->  8.7       13.0 ->  7.3       14.8 -> 14.1*      17.4 -> 11.3
+//     300  15.1 -> 13.4*      14.7 -> 10.6       30.2 -> 21.5*      19.7 -> 17.2
+//     512  16.1 -> 14.6*      15.3 -> 12.4       31.6 -> 28.8*      22.3 -> 22.3*
 #include <hip/hip_fp16.h>
 
 #include "qlin_epilogue.hpp"
@@ -292,12 +292,12 @@ static hipError_t launch_c(const GemmParams& p, int bits, hipStream_t st) {
 // Tile configurations: row fragments MF and channel blocks NB of 16, waves WK along k, stages R of a
 // wave's ring (as many as fit 160 KiB, at most what the shortest K uses), time against the planner's
 // estimate (W4, W8).
-#define QLIN_KS_CONFIGS(X)                                                                                             \
-    X(0, 1, 1, 4, 6, 1.02, 0.99) X(1, 1, 1, 8, 4, 1, 1.02) X(2, 1, 2, 4, 4, 0.97, 0.98) X(3, 1, 3, 4, 4, 0.98, 1.01)   \
-    X(4, 1, 6, 4, 4, 1.05, 0.99) X(5, 2, 1, 4, 4, 1.02, 0.98) X(6, 2, 2, 4, 4, 1, 1) X(7, 2, 3, 4, 3, 0.99, 0.98)      \
-    X(8, 2, 3, 8, 2, 0.93, 1) X(9, 2, 4, 4, 3, 0.98, 0.99) X(10, 2, 6, 4, 4, 1.01, 0.98) X(11, 3, 2, 4, 3, 0.99, 0.98) \
-    X(12, 3, 2, 8, 2, 0.94, 1) X(13, 3, 3, 4, 3, 1.02, 1) X(14, 4, 3, 4, 3, 1.02, 0.97) X(15, 4, 4, 4, 3, 1.02, 0.98)  \
-    X(16, 4, 5, 4, 2, 1, 1) X(17, 4, 6, 4, 2, 1.01, 1) X(18, 6, 3, 4, 2, 1.04, 1.02) X(19, 6, 4, 4, 2, 1.01, 1)
+#define QLIN_KS_CONFIGS(X)                                                                                              \
+    X(0, 1, 1, 4, 6, 1.02, 1.01) X(1, 1, 1, 8, 4, 1, 1.03) X(2, 1, 2, 4, 4, 0.97, 0.99) X(3, 1, 3, 4, 4, 0.98, 1.01)    \
+    X(4, 1, 6, 4, 4, 1.03, 0.98) X(5, 2, 1, 4, 4, 1.03, 0.99) X(6, 2, 2, 4, 4, 1.01, 1.01) X(7, 2, 3, 4, 3, 0.99, 0.98) \
+    X(8, 2, 3, 8, 2, 0.93, 1) X(9, 2, 4, 4, 3, 0.98, 0.99) X(10, 2, 6, 4, 4, 0.99, 0.97) X(11, 3, 2, 4, 3, 1, 0.99)     \
+    X(12, 3, 2, 8, 2, 0.94, 1) X(13, 3, 3, 4, 3, 1.01, 0.99) X(14, 4, 3, 4, 3, 1.02, 0.96) X(15, 4, 4, 4, 3, 1, 0.96)   \
+    X(16, 4, 5, 4, 2, 0.97, 0.98) X(17, 4, 6, 4, 2, 0.96, 1) X(18, 6, 3, 4, 2, 1.02, 1.01) X(19, 6, 4, 4, 2, 0.99, 1)
 
 KsTile gemm_ks_tile(int cfg) {
     switch (cfg) {

@@ -363,14 +363,14 @@ static hipError_t launch_c(const GemmParams& p, int cus, hipStream_t st) {
 // (each wave then needs an even number of 16-row blocks).
 constexpr PpTile kPpTiles[kPpConfigs] = {
     // bm, bn, W4, W8, plain, SiLU-gate, us per k step W4, W8, us per tile W4, W8
-    {256, 256, true, false, false, true, {1.03, 0}, {5.91, 0}},
-    {256, 192, true, false, true, true, {0.867, 0}, {4.61, 0}},
-    {256, 128, true, true, true, true, {0.562, 0.559}, {3.3, 3.09}},
-    {128, 96, true, true, true, false, {0.329, 0.332}, {1.92, 2.01}},
-    {128, 128, true, true, true, true, {0.355, 0.37}, {1.81, 1.74}},
-    {128, 192, true, true, true, false, {0.45, 0.505}, {3.16, 2.62}},
-    {128, 192, true, true, false, true, {0.512, 0.52}, {3.18, 2.47}},
-    {128, 256, true, true, true, true, {0.582, 0.607}, {3.53, 3.16}},
+    {256, 256, true, false, false, true, {1.03, 0}, {5.63, 0}},
+    {256, 192, true, false, true, true, {0.856, 0}, {4.54, 0}},
+    {256, 128, true, true, true, true, {0.553, 0.574}, {3.24, 3.11}},
+    {128, 96, true, true, true, false, {0.32, 0.348}, {1.95, 1.97}},
+    {128, 128, true, true, true, true, {0.349, 0.383}, {1.84, 1.75}},
+    {128, 192, true, true, true, false, {0.447, 0.527}, {3.2, 2.62}},
+    {128, 192, true, true, false, true, {0.505, 0.534}, {3.15, 2.48}},
+    {128, 256, true, true, true, true, {0.576, 0.632}, {3.53, 3.19}},
 };
 
 PpTile gemm_pp_tile(int cfg) { return kPpTiles[cfg]; }
